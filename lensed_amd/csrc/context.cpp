@@ -312,7 +312,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         if (!S.psfw || S.sep_rank != 1 || S.psfw > LENSED_SWEEP_MAX_PSF || S.psfh > LENSED_SWEEP_MAX_PSF ||
             S.height > LENSED_SWEEP_MAX_H)
             sweep_ok = false;
-        if (!(S.table && S.cull && !(l->flags & LENSED_NO_CULL))) all_culled = false;
+        if (!S.cull || (l->flags & LENSED_NO_CULL)) all_culled = false;
     }
     if (!tq.conv_rows && sweep_ok && all_culled) L.conv_rows = LENSED_CONV_SWEEP;
     if (L.conv_rows == LENSED_CONV_SWEEP && !sweep_ok)
@@ -382,9 +382,9 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         d.sep_rank = S.sep_rank;
         d.sep_off = S.sep_off;
         d.psft_off = S.psft_off;
-        d.npre_off = S.table ? npre_off : 0;
+        d.npre_off = npre_off;
         d.qrad = S.qrad;
-        d.cull = S.table && S.cull && !(l->flags & LENSED_NO_CULL) ? 1 : 0;
+        d.cull = S.cull && !(l->flags & LENSED_NO_CULL) ? 1 : 0;
         d.dark_off = S.dark_off;
         L.any_cull = L.any_cull || d.cull;
         long long nc = (long long)ncand[s];
@@ -398,8 +398,8 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         ic += (int)(nc * (sweep ? d.tiles_x : d.ntile_c));  // sweep: one item per 64-column strip
         is += (int)nc;
         iff += (int)nc;
+        if (S.table || S.cull) npre_off += nc * LENSED_NPRE_STRIDE(S.table ? S.nq : 0);
         if (S.table) {
-            npre_off += nc * LENSED_NPRE_STRIDE(S.nq);
             table_off += nc * LENSED_EPL_TABLE_F4;
             itab += (int)(nc * LENSED_EPL_ROWS);
             inode += (int)(nc * LENSED_EPL_ROWS);
@@ -926,7 +926,7 @@ lensed* lensed_create(const lensed_system* systems, size_t nsys, const lensed_op
         }
         fast_priors(S);
         S.dwords = model_data_words(S.objs);
-        S.cull = S.table && model_culls(S.objs);
+        S.cull = model_culls(S.objs);
         // model index: identical object lists share one compute function
         int model = -1;
         for (size_t k = 0; k < models.size() && model < 0; ++k) {
@@ -1058,7 +1058,7 @@ lensed* lensed_create(const lensed_system* systems, size_t nsys, const lensed_op
         l->cap_partials += l->max_batch * ((S.height + 7) / 8) * ((S.width + LENSED_CONV_TX - 1) / LENSED_CONV_TX);
         l->cap_out += l->max_batch;
         if (S.table) l->cap_tables += l->max_batch * LENSED_EPL_TABLE_F4;
-        if (S.table) l->cap_npre += l->max_batch * LENSED_NPRE_STRIDE(S.nq);
+        if (S.table || S.cull) l->cap_npre += l->max_batch * LENSED_NPRE_STRIDE(S.table ? S.nq : 0);
         l->cap_trace += l->max_batch * S.ntile_r * (LENSED_RENDER_BS / 64);
         l->cap_cull += l->max_batch * ((S.ntile_r + LENSED_CULL_GROUP - 1) / LENSED_CULL_GROUP);
     }
@@ -1498,7 +1498,7 @@ int lensed_loglike_batch_noalloc(lensed* l, size_t s, const double* cubes, size_
     const size_t sizes[] = {sizeof(lensed_desc),
                             nc * d.npar * 4,
                             (nc * d.dwords + 256) * 4,
-                            d.table_mode ? nc * LENSED_NPRE_STRIDE(d.nq) * 16 : 16,
+                            d.table_mode || S.cull ? nc * LENSED_NPRE_STRIDE(d.table_mode ? d.nq : 0) * 16 : 16,
                             d.table_mode ? nc * LENSED_EPL_TABLE_F4 * 16 : 16,
                             nc * (size_t)d.npix * 4,
                             nc * (size_t)d.npart * 8,

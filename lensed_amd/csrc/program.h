@@ -63,7 +63,8 @@ bool object_table_shear(const std::string& name);
 // set_params_<k>().  Offsets are in 4-byte words.
 std::string compute_function(const std::vector<ModelObject>& objs, int k);
 // whether the model's pixels can be culled before the render: a tabulated
-// EPL lens and one source with a frame and a cutoff, nothing else
+// EPL lens and one source with a frame and a cutoff, nothing else; or lenses
+// that bound their own slope (deflection_slope), then compact sources
 bool model_culls(const std::vector<ModelObject>& objs);
 std::string set_params_function(const std::vector<ModelObject>& objs, int k);
 

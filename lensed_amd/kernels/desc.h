@@ -29,9 +29,10 @@
 // rows are contiguous (16-byte stride), so lanes reading nearby rows hit
 // different LDS banks
 #define LENSED_EPL_AT(comp, i) ((comp) * LENSED_EPL_ROWS + (i))
-// per candidate in npre[]: the nq node pairs, then the pixel cull's constants
+// per candidate in npre[]: the node pairs of a tabulated lens (nq of them,
+// none without a table), then the pixel cull's constants
 #define LENSED_NPRE_CULL 3
-#define LENSED_NPRE_STRIDE(nq) ((nq) + LENSED_NPRE_CULL)
+#define LENSED_NPRE_STRIDE(pairs) ((pairs) + LENSED_NPRE_CULL)
 
 struct lensed_desc {
     int width, height, npix, model;  // image size, pixels, model index
@@ -54,7 +55,7 @@ struct lensed_desc {
                                             // in use; first emulator node item (NT + 1 nodes per candidate);
                                             // first cull item (LENSED_CULL_GROUP render items each)
     long long psft_off;                  // floats into psf[]: the taps transposed, [psfw][psfh]
-    long long npre_off;                  // float4 into npre[]: node pairs, cull constants ([ncand][nq + 3])
+    long long npre_off;                  // float4 into npre[]: node pairs, cull constants ([ncand][pairs + 3])
     float qrad;                          // largest distance of a quadrature node from the pixel centre
     int cull;                            // skip pixels whose rays provably all miss the source
     long long dark_off;                  // doubles into the data's chi^2 block partials for a model of 0 ([npart])

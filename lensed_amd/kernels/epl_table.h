@@ -170,6 +170,23 @@ inline bool lensed_frame_cull(const D* self, float4 base, const float4* tab, con
     return rlo > 0.0f && sqrtf(us.x * us.x + us.y * us.y) - d > b.w;
 }
 
+// The same proof in the image frame, for lenses without a table that bound
+// their own slope (deflection_slope: the operator norm of the deflection's
+// derivative over the disc of radius rho): every ray of the pixel lands within
+// rho (1 + sum of slopes) of the centre ray, in the source's frame within |T|
+// times that of u.  The margin is the lens-frame form's 1/16 unit plus
+// 2^-8 pixels, for the FP32 rounding of the ray positions themselves (formed
+// from image coordinates of up to thousands of pixels).
+inline float2 lensed_slope_cull_consts(float2 t0, float2 t1, float cutoff) {
+    const float tn = sqrtf(dot(t0, t0) + dot(t1, t1));
+    return float2(tn, cutoff + 0.0625f + 0.00390625f * tn);
+}
+
+// (an infinite or NaN slope compares false: the pixel is kept)
+inline bool lensed_slope_cull(float2 u, float tn, float cutoff, float rho, float slope) {
+    return sqrtf(u.x * u.x + u.y * u.y) - tn * rho * slope > cutoff;
+}
+
 }  // namespace lcl
 #ifdef LCL_GPU
 #pragma clang force_cuda_host_device end

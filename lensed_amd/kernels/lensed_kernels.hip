@@ -66,15 +66,16 @@ __device__ inline void lensed_node_pairs(const lensed_desc& d, u32* blk, const f
                                          float4* __restrict__ npre, int cand)
 {
     const float4* q = quad + d.quad_off;
-    float4* out = npre + d.npre_off + (long long)cand * LENSED_NPRE_STRIDE(d.nq);
-    for (int n = 0; n < d.nq; ++n) {
+    const int pairs = d.table_mode ? d.nq : 0;
+    float4* out = npre + d.npre_off + (long long)cand * LENSED_NPRE_STRIDE(pairs);
+    for (int n = 0; n < pairs; ++n) {
         lcl::float4 v = lcl::epl_pre_model<K>(blk, lcl::float2(q[n].x, q[n].y), false);
         out[n] = make_float4(v.x, v.y, v.z, v.w);
     }
-    if (d.cull) {  // the candidate's constants of the pixel cull (lensed_frame_cull)
+    if (d.cull) {  // the candidate's constants of the pixel cull
         lcl::float4 cc[LENSED_NPRE_CULL];
         lcl::cull_consts_model<K>(blk, cc);
-        for (int i = 0; i < LENSED_NPRE_CULL; ++i) out[d.nq + i] = make_float4(cc[i].x, cc[i].y, cc[i].z, cc[i].w);
+        for (int i = 0; i < LENSED_NPRE_CULL; ++i) out[pairs + i] = make_float4(cc[i].x, cc[i].y, cc[i].z, cc[i].w);
     }
 }
 
@@ -103,7 +104,8 @@ __device__ __attribute__((always_inline)) inline void lensed_set_params_item(
 #define LENSED_SET_CASE(K)                                                \
     case K:                                                               \
         lcl::set_params_##K(blk, p);                                      \
-        if (d.table_mode) lensed_node_pairs<K>(d, blk, quad, npre, cand); \
+        if (d.table_mode || d.cull)                                       \
+            lensed_node_pairs<K>(d, blk, quad, npre, cand);               \
         break;
         LENSED_FOR_MODELS(LENSED_SET_CASE)
 #undef LENSED_SET_CASE
@@ -267,8 +269,8 @@ extern "C" __global__ __launch_bounds__(LENSED_RENDER_BS) __attribute__((amdgpu_
 // -------------------------------------------------------------------- cull
 // Before the render: for each 8 x 8 square of each render item (a wave's
 // pixels in the render's walk), and for each 4 x 4 quad of a square, whether
-// any of its pixels can receive light (lensed_frame_cull in epl_table.h
-// bounds where a pixel's rays land).  Dark quads get their zero model values
+// any of its pixels can receive light (cull_<k>, generated for the
+// model, bounds where a pixel's rays land).  Dark quads get their zero model values
 // here (where they may be missing) and are left out of the render; the lit
 // ones go to a list that the render's blocks share out evenly, four quads to
 // a wave (lit quads bunch in the middle of the image, so a fixed
@@ -280,9 +282,10 @@ extern "C" __global__ __launch_bounds__(LENSED_RENDER_BS) __attribute__((amdgpu_
 // A cull work item is LENSED_CULL_GROUP render items of one candidate: 256
 // squares, 64 to each wave, which settles its own squares without waiting
 // for the others; a block takes consecutive items and stages a candidate's
-// table once for all.  Only systems with d.cull (a tabulated EPL lens and one
-// framed source with a cutoff) are tested; the quads of the others are all
-// listed.
+// table once for all.  Only systems with d.cull are tested (a tabulated EPL
+// lens and one framed source with a cutoff, lensed_frame_cull; or lenses that
+// bound their own slope and compact sources, the generated cull_<k>); the
+// quads of the others are all listed.
 static_assert(LENSED_RENDER_BS == 256 && LENSED_CULL_GROUP == 64, "a cull item gives each wave 64 squares");
 
 // lanes (pixels y * 8 + x of a square) of its quad q = 2 * (y / 4) + x / 4
@@ -301,7 +304,8 @@ __device__ inline int lensed_cull_wave(const lensed_desc& d, int cand, int g0, i
     const u32* gb = blocks + d.block_off + (long long)cand * d.dwords;
 #pragma unroll
     for (int i = 0; i < LENSED_DWORDS; ++i) blk[i] = i < d.dwords ? __builtin_amdgcn_readfirstlane(gb[i]) : 0u;
-    const float4* ccg = npre + d.npre_off + (long long)cand * LENSED_NPRE_STRIDE(d.nq) + d.nq;
+    const int pairs = d.table_mode ? d.nq : 0;
+    const float4* ccg = npre + d.npre_off + (long long)cand * LENSED_NPRE_STRIDE(pairs) + pairs;
     lcl::float4 cc[LENSED_NPRE_CULL];
 #pragma unroll
     for (int i = 0; i < LENSED_NPRE_CULL; ++i) cc[i] = lcl::float4(ccg[i].x, ccg[i].y, ccg[i].z, ccg[i].w);
@@ -488,7 +492,7 @@ extern "C" __global__ __launch_bounds__(LENSED_RENDER_BS) void lensed_cull(
         const int sq = wave * 64 + lane;              // this lane's square of the item
         if (key != staged) {
             pad();  // entries never mix candidates
-            if (d.cull) {
+            if (d.cull && d.table_mode) {
                 __syncthreads();  // no wave reads the previous candidate's table any more
                 const float4* src = tables + d.table_off + (long long)cand * LENSED_EPL_TABLE_F4;
                 for (int i = threadIdx.x; i < LENSED_EPL_TABLE_F4; i += LENSED_RENDER_BS) tab_lds[i] = src[i];

@@ -43,6 +43,28 @@ static float2 deflection(local data* this, float2 x)
     return mv22(this->bwd, powr(uu, this->hexp)*sum);
 }
 
+// bound on the deflection's slope (operator norm) within rho of x: with
+// |u| >= lo there, |bwd| |u|^(-t) (|1-t| A + B) |fwd|, A = sum |C_k| and
+// B = sum (2k+1) |C_k| the bounds of the series and its derivative, and
+// Frobenius norms; infinite where the disc may hold the centre
+static float deflection_slope(local data* this, float2 x, float rho)
+{
+    float2 d = x - this->c;
+    float2 u = mv22(this->fwd, d);
+    float fr = sqrt(dot(this->fwd, this->fwd))*rho;
+    float r = length(u);
+    float t = 1 - 2*this->hexp;
+    float a = 1;
+    float b = 1;
+    for(int k = 0; k < 10; ++k)
+    {
+        a += fabs(this->coef[k]);
+        b += (2*k + 3)*fabs(this->coef[k]);
+    }
+    float s = sqrt(dot(this->bwd, this->bwd)*dot(this->fwd, this->fwd))*(fabs(1 - t)*a + b);
+    return r > fr ? s*exp2(-t*log2(t > 0 ? r - fr : r + fr)) : HUGE_VALF;
+}
+
 static void set(local data* this, float x, float y, float r, float t, float q, float pa)
 {
     float cs;

@@ -43,6 +43,12 @@ static float frame_cutoff(local data* this)
     return sqrt(fmax(this->lpk + 127, 0.0f));
 }
 
+// the cutoff is about 13 sigma out: most pixels of an image lie beyond it
+static bool frame_compact(local data* this)
+{
+    return true;
+}
+
 static float brightness(local data* this, float2 x)
 {
     return frame_profile(this, frame_map(this, x - frame_centre(this)));

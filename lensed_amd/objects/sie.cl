@@ -29,6 +29,17 @@ static float2 deflection(local data* this, float2 x)
     return mv22(this->bwd, this->amp*(float2)(atan(u.x*s), atanh(u.y*s)));
 }
 
+// bound on the deflection's slope (operator norm) within rho of x: its
+// derivative has eigenvalues 0 and 2 kappa = r sqrt(q)/w, and w changes by at
+// most rho; infinite where the disc may hold the centre
+static float deflection_slope(local data* this, float2 x, float rho)
+{
+    float2 d = x - this->c;
+    float2 u = mv22(this->fwd, d);
+    float w = sqrt(this->qq*u.x*u.x + u.y*u.y) - rho;
+    return w > 0 ? this->amp*this->ecc/w : HUGE_VALF;
+}
+
 static void set(local data* this, float x, float y, float r, float q, float pa)
 {
     float cs = cos(pa*DEG2RAD);

@@ -1,0 +1,148 @@
+"""The image-frame pixel cull of models without a tabulated lens: lenses that
+bound their own slope (deflection_slope) and compact sources (frame_compact).
+
+On the CPU the generated model code is compiled for the host and every ray of
+every skipped pixel traced; on the GPU culled launches must give the bits of
+tracing every ray."""
+import ctypes
+import os
+import subprocess
+import tempfile
+from ctypes import POINTER, c_float, c_int
+
+import numpy as np
+import pytest
+
+from host_model import load_objects
+from lensed_amd import _lib as L
+from lensed_amd import quadrature as Q
+from lensed_amd import workloads as W
+from lensed_amd._lib import LENSED_GRAPH, LENSED_NO_CULL
+from lensed_amd.lensed import Context, SystemSpec
+
+HARNESS = r'''
+// pixels the cull skips, and how many of their rays give a normal (not
+// subnormal: the kernels flush those to 0) brightness
+extern "C" void host_cull(const float* params, int w, int h, const float* q, int nq, float rho, int* out) {
+    static lcl::uint data[4096];
+    lcl::set_params_0(data, params);
+    lcl::float4 cc[LENSED_NPRE_CULL];
+    lcl::cull_consts_0(data, cc);
+    out[0] = out[1] = 0;
+    for (int k = 0; k < w * h; ++k) {
+        const float cx = 1.0f + (float)(k % w), cy = 1.0f + (float)(k / w);
+        if (!lcl::cull_0(data, lcl::epl_pre_0(data, lcl::float2(cx, cy), true), nullptr, cc, rho)) continue;
+        ++out[0];
+        for (int n = 0; n < nq; ++n)
+            out[1] += !(std::fabs(lcl::compute_0(data, lcl::float2(cx + q[2 * n], cy + q[2 * n + 1]), nullptr)) <
+                        FLT_MIN);
+    }
+}
+'''
+
+LENS = {"epl": ("x", "y", "r", "t", "q", "pa"), "epl_plus_shear": ("x", "y", "r", "t", "q", "pa", "g1", "g2"),
+        "sie": ("x", "y", "r", "q", "pa"), "sie_plus_shear": ("x", "y", "r", "q", "pa", "g1", "g2")}
+GAUSS = ("x", "y", "sigma", "mag", "q", "pa")
+
+
+def _host(objects):
+    arr = load_objects(objects)
+    src = L.take_string(L.load().lensed_model_source(len(objects), arr)) + HARNESS
+    assert "lensed_slope_cull(" in src.split("cull_0", 1)[1]
+    d = tempfile.mkdtemp(prefix="lensed_slope_")
+    cpp, so = os.path.join(d, "m.cpp"), os.path.join(d, "m.so")
+    open(cpp, "w").write(src)
+    subprocess.check_call(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-w", "-o", so, cpp])
+    lib = ctypes.CDLL(so)
+    fp = POINTER(c_float)
+    lib.host_cull.argtypes = [fp, c_int, c_int, fp, c_int, c_float, POINTER(c_int)]
+    return lib
+
+
+@pytest.mark.parametrize("lens", list(LENS))
+@pytest.mark.parametrize("nsrc", [1, 3])
+def test_slope_cull_never_skips_a_lit_ray(lens, nsrc):
+    lib = _host([("lens", lens)] + [("s%d" % i, "gauss") for i in range(nsrc)])
+    qq, _ = Q.rule("g3k7")
+    qn = np.ascontiguousarray(np.asarray(qq, np.float32).reshape(-1, 2))
+    rng = np.random.default_rng(21)
+    fp = POINTER(c_float)
+    out = (c_int * 2)()
+    skipped = 0
+    for it in range(14):
+        v = {"x": rng.uniform(45, 56), "y": rng.uniform(45, 56), "r": rng.uniform(5, 15), "t": rng.uniform(0.3, 1.7),
+             "q": rng.uniform(0.1, 1.0) if it % 5 else 1.0, "pa": rng.uniform(0, 180), "g1": rng.uniform(-0.2, 0.2),
+             "g2": rng.uniform(-0.2, 0.2)}
+        if it % 4 == 0:
+            v["x"], v["y"] = 50.0, 50.0  # the lens centre on a pixel centre
+        params = [v[p] for p in LENS[lens]]
+        for _ in range(nsrc):
+            s = {"x": rng.uniform(40, 60), "y": rng.uniform(40, 60), "sigma": 10 ** rng.uniform(-1, 0.5),
+                 "mag": rng.uniform(-8, 5), "q": rng.uniform(0.3, 1), "pa": rng.uniform(0, 180)}
+            params += [s[p] for p in GAUSS]
+        params = np.array(params, np.float32)
+        # the pixel's own rays, and the quads and squares of pixels as the cull tests them
+        for grow in (0.0, 1.5, 3.5):
+            box = np.arange(-grow, grow + 0.5, 1.0, dtype=np.float32)
+            q = np.concatenate([qn + np.array([dx, dy], np.float32) for dx in box[[0, -1]] for dy in box[[0, -1]]])
+            rho = float(np.hypot(qn[:, 0], qn[:, 1]).max() * (1 + 1e-6) + grow * np.sqrt(2))
+            lib.host_cull(params.ctypes.data_as(fp), 100, 100, np.ascontiguousarray(q).ctypes.data_as(fp), len(q),
+                          rho, out)
+            assert out[1] == 0, (it, grow, params, list(out))
+            skipped += out[0]
+    assert skipped > 1000, skipped
+
+
+def test_models_that_take_the_slope_cull():
+    """Lenses first, then compact sources alone; anything else (a sky, a
+    source with a far cutoff, a source before the lens, a lens without a
+    bound) traces every ray."""
+    def culls(*objects):
+        objs = [("o%d" % i, n) for i, n in enumerate(objects)]
+        src = L.take_string(L.load().lensed_model_source(len(objs), load_objects(objs)))
+        return "lensed_slope_cull(" in src.split("cull_0", 1)[1]
+    assert culls("sie", "gauss") and culls("epl", "sie_plus_shear", "gauss", "gauss")
+    assert not culls("sie", "sersic") and not culls("sie", "gauss", "sky") and not culls("nsie", "gauss")
+    assert not culls("gauss", "sie", "gauss") and not culls("gauss") and not culls(*["sie"] + ["gauss"] * 7)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,nsrc,shape,psf", [("epl_plus_shear", 1, (131, 97), (21, 21)), ("sie", 2, (64, 64), (5, 8)),
+                                                  ("epl", 1, (48, 203), None), ("sie_plus_shear", 3, (90, 33), (31, 9))])
+def test_slope_cull_keeps_the_bits(lens, nsrc, shape, psf):
+    h, w = shape
+    rng = np.random.default_rng(h * w)
+    cx, cy, r = (w + 1) / 2, (h + 1) / 2, min(h, w) / 8
+    span = {"x": (cx - 2, cx + 2), "y": (cy - 2, cy + 2), "r": (0.7 * r, 1.3 * r), "t": (0.5, 1.5), "q": (0.3, 1),
+            "pa": (0, 180), "g1": (-0.1, 0.1), "g2": (-0.1, 0.1), "sigma": (0.05 * r, 0.15 * r), "mag": (-5, 5)}
+    pri = {f"lens.{p}": "unif %g %g" % span[p] for p in LENS[lens]}
+    for i in range(nsrc):
+        pri.update({f"s{i}.{p}": "unif %g %g" % span[p] for p in GAUSS})
+    taps = None
+    if psf:
+        n = max(psf)
+        taps = W.gaussian_psf(n, 3.0)[(n - psf[0]) // 2:(n - psf[0]) // 2 + psf[0],
+                                      (n - psf[1]) // 2:(n - psf[1]) // 2 + psf[1]].copy()
+        taps /= taps.sum()
+    image = rng.normal(0, 0.05, shape).astype(np.float32)
+    res = []
+    for extra in (0, LENSED_NO_CULL):
+        spec = SystemSpec([("lens", lens)] + [(f"s{i}", "gauss") for i in range(nsrc)], pri, image,
+                          np.full(shape, 400.0, np.float32), psf=taps)
+        with Context(spec, max_batch=300, flags=LENSED_GRAPH | extra) as ctx:
+            g = np.random.default_rng(3)
+            first, second = g.random((300, ctx.ndims())), g.random((300, ctx.ndims()))
+            l1, p1 = ctx.loglike_batch(first)
+            items, kept, quads, _ = ctx.render_stats()
+            l2, _ = ctx.loglike_batch(second)  # the cull trusts its record of the first launch's quads
+            phys = np.zeros(ctx.npars())
+            phys[ctx.pmap()] = p1[0]
+            res.append((l1, l2, ctx.render(phys), ctx.loglike(first[5])[0]))
+        if not extra:
+            assert quads < 16 * items, (items, kept, quads)
+        else:
+            assert quads == 16 * items
+    (a1, a2, ap, al), (b1, b2, bp, bl) = res
+    assert np.all(np.isfinite(a1)) and np.array_equal(a1, b1) and np.array_equal(a2, b2) and al == bl
+    for k in ap:
+        assert np.array_equal(ap[k], bp[k]), k
