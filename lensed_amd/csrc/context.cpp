@@ -303,18 +303,27 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
     // PSF of at most 21 x 21, and at most 512 rows.  It is the default
     // where every such system is also culled: it skips the rows the cull
     // found dark, and with every row lit the tile is the faster (C3 at 4096
-    // candidates: 0.50 against 0.85 ms; C4, nothing culled: 14.0 against
-    // 8.0 ms)
+    // candidates: 0.30 against 0.80 ms; C4, nothing culled: 14.0 against
+    // 8.0 ms), from two strips per CU on.  A wave takes about 0.25 us per row
+    // of its strip whatever else runs, so fewer strips leave the device
+    // waiting for a few waves (256 x 256, 21 x 21 PSF, sweep with each strip
+    // cut as below against the tile: 1 candidate 16 / 8 us, 16: 17 / 12, 64:
+    // 24 / 19, 128: 34 / 33, 256: 41 / 55, 512: 68 / 111), and up to four
+    // waves per SIMD each strip is cut into parts, a wave each, at the price
+    // of refilling the window above every part (256 candidates whole, in 2, 4
+    // and 8 parts: 70, 45, 41 and 50 us; 1024: 93, 92, 112 and 126).
     bool sweep_ok = true, all_culled = true;
+    long long strips = 0;
     for (size_t s = 0; s < l->sys.size(); ++s) {
         const System& S = l->sys[s];
         if (!ncand[s]) continue;
+        strips += (long long)ncand[s] * ((S.width + 63) / 64);
         if (!S.psfw || S.sep_rank != 1 || S.psfw > LENSED_SWEEP_MAX_PSF || S.psfh > LENSED_SWEEP_MAX_PSF ||
             S.height > LENSED_SWEEP_MAX_H)
             sweep_ok = false;
         if (!S.cull || (l->flags & LENSED_NO_CULL)) all_culled = false;
     }
-    if (!tq.conv_rows && sweep_ok && all_culled) L.conv_rows = LENSED_CONV_SWEEP;
+    if (!tq.conv_rows && sweep_ok && all_culled && strips >= 2LL * l->cu_count) L.conv_rows = LENSED_CONV_SWEEP;
     if (L.conv_rows == LENSED_CONV_SWEEP && !sweep_ok)
         L.conv_rows = L.conv_small ? LENSED_CONV_RY_SMALL : LENSED_CONV_RY;
     if (L.conv_rows == LENSED_CONV_RY_TALL) {
@@ -329,6 +338,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
     }
     L.conv_small = L.conv_rows == LENSED_CONV_RY_SMALL;
     const bool sweep = L.conv_rows == LENSED_CONV_SWEEP;
+    const int seg = (int)std::min(64LL, std::max(1LL, (16LL * l->cu_count + strips - 1) / strips));
     const int ry = sweep ? LENSED_CONV_RY : L.conv_rows;  // (tile counts of a sweep layout are not used)
     const int th = LENSED_CONV_TY * ry;
     long long param_off = 0, block_off = 0, model_off = 0, partial_off = 0, out_off = 0, table_off = 0;
@@ -386,6 +396,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         d.qrad = S.qrad;
         d.cull = S.cull && !(l->flags & LENSED_NO_CULL) ? 1 : 0;
         d.dark_off = S.dark_off;
+        d.sweep_seg = seg;
         L.any_cull = L.any_cull || d.cull;
         long long nc = (long long)ncand[s];
         param_off += nc * d.npar;
@@ -395,7 +406,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         out_off += nc;
         ir += (int)(nc * d.ntile_r);
         ik += (int)(nc * ((d.ntile_r + LENSED_CULL_GROUP - 1) / LENSED_CULL_GROUP));
-        ic += (int)(nc * (sweep ? d.tiles_x : d.ntile_c));  // sweep: one item per 64-column strip
+        ic += (int)(nc * (sweep ? d.tiles_x * seg : d.ntile_c));  // sweep: an item per part of a 64-column strip
         is += (int)nc;
         iff += (int)nc;
         if (S.table || S.cull) npre_off += nc * LENSED_NPRE_STRIDE(S.table ? S.nq : 0);
@@ -1544,7 +1555,7 @@ int lensed_loglike_batch_noalloc(lensed* l, size_t s, const double* cubes, size_
     L.n_set = L.n_final = n;
     L.n_render = n * d.ntile_r;
     L.n_cull = n * ((d.ntile_r + LENSED_CULL_GROUP - 1) / LENSED_CULL_GROUP);
-    L.n_conv = n * (L.conv_rows == LENSED_CONV_SWEEP ? d.tiles_x : d.ntile_c);
+    L.n_conv = n * (L.conv_rows == LENSED_CONV_SWEEP ? d.tiles_x * d.sweep_seg : d.ntile_c);
     L.n_table = L.n_nodes = d.table_mode ? n * LENSED_EPL_ROWS : 0;
     L.n_tcands = d.table_mode ? n : 0;
     {

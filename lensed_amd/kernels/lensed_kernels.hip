@@ -1057,8 +1057,9 @@ extern "C" __global__ __launch_bounds__(LENSED_CONV_BS) __attribute__((amdgpu_wa
 
 // ------------------------------------------------------ conv+chi2, sweep
 // Rank-1 separable PSFs of at most 21 x 21, images up to 512 rows (the
-// host checks both): one wave per 64-column strip
-// of one candidate's image sweeps the strip from top to bottom.  Per input
+// host checks both): one wave per 64-column strip of one candidate's image
+// sweeps the strip from top to bottom (d.sweep_seg waves, each an equal part
+// of its lit rows, where a launch has few strips).  Per input
 // row, the row pass of the strip's 64 columns, from the row and its PSF halo
 // staged in the wave's LDS row, goes into a window of the last PH row-pass
 // values per lane (registers; the sweep is unrolled PH rows at a time, so
@@ -1077,7 +1078,7 @@ extern "C" __global__ __launch_bounds__(LENSED_CONV_BS) __attribute__((amdgpu_wa
 #define LENSED_SWEEP_ROW 96  // floats per wave's staged row: 64 + PW - 1 for PW <= LENSED_SWEEP_MAX_PSF
 
 template <int PW, int PH, bool OUT>
-__device__ inline void lensed_conv_sweep_item(const lensed_desc& d, int cand, int strip,
+__device__ inline void lensed_conv_sweep_item(const lensed_desc& d, int cand, int strip, int seg,
                                               const float* __restrict__ model, const float* __restrict__ image,
                                               const float* __restrict__ weight, const float* __restrict__ psf,
                                               double* __restrict__ partials, float* __restrict__ conv_out,
@@ -1148,11 +1149,19 @@ __device__ inline void lensed_conv_sweep_item(const lensed_desc& d, int cand, in
     // (wave-uniform, and known so: the sweep's row counters stay scalar)
     first = __builtin_amdgcn_readfirstlane(first);
     stop = __builtin_amdgcn_readfirstlane(stop);
-    if (skip && lane < nblk && (lane < first || lane >= stop))
+    if (skip && seg == 0 && lane < nblk && (lane < first || lane >= stop))
         part[(long long)lane * d.tiles_x] = dark[d.dark_off + (long long)lane * d.tiles_x + strip];
+    // this wave's share of the swept blocks (its first windows are refilled
+    // from the PH - 1 rows above, so any split gives the same bits)
+    {
+        const int n = stop - first;
+        stop = first + n * (seg + 1) / d.sweep_seg;
+        first += n * seg / d.sweep_seg;
+        if (first >= stop) return;
+    }
     const int y_first = 8 * first;                          // first output row swept
     const int yi0 = max(y_first + A - (PH - 1), 0);         // first input row its window reads
-    const int yi_end = stop > first ? min(8 * stop, H) + A : yi0;  // input rows [yi0, yi_end)
+    const int yi_end = min(8 * stop, H) + A;                // input rows [yi0, yi_end)
     // Loads, issued four iterations ahead in iteration order so that the
     // counter waits keep four iterations in flight; every address is a fixed
     // base plus a wave-uniform row offset plus the lane's byte offset.  Model
@@ -1265,7 +1274,8 @@ __device__ inline void lensed_conv_sweep_item(const lensed_desc& d, int cand, in
     }
 }
 
-// One wave per item (a 64-column strip of one candidate), four per block.
+// One wave per item (a 64-column strip of one candidate, or a part of one,
+// the parts of a strip side by side), four per block.
 // Blocks go to the eight XCDs in turn; XCD x takes the x-th contiguous share
 // of the blocks, so the strips of a candidate run side by side in one L2,
 // which holds the halo columns that neighbouring strips both read.  The
@@ -1292,7 +1302,8 @@ __device__ inline void lensed_conv_sweep_body(const lensed_desc* __restrict__ sy
     const int s = lensed_find_sys<1>(sys, nsys, item);
     const lensed_desc& d = sys[s];
     const int local = item - d.item_c;
-    const int cand = local / d.tiles_x, strip = local - cand * d.tiles_x;
+    const int seg = local % d.sweep_seg, col = local / d.sweep_seg;
+    const int cand = col / d.tiles_x, strip = col - cand * d.tiles_x;
     float* lrow = rows + wave * LENSED_SWEEP_ROW;
     // (the host launches the sweep only for layouts whose PSFs are all
     // separable and at most LENSED_SWEEP_MAX_PSF on a side; the others are
@@ -1300,7 +1311,7 @@ __device__ inline void lensed_conv_sweep_body(const lensed_desc* __restrict__ sy
 #define LENSED_SWEEP_CASE(PW_, PH_, SEP_)                                                                 \
     if constexpr (SEP_ && PW_ <= LENSED_SWEEP_MAX_PSF && PH_ <= LENSED_SWEEP_MAX_PSF) {                 \
         if (d.psfw == PW_ && d.psfh == PH_) {                                                           \
-            lensed_conv_sweep_item<PW_, PH_, OUT>(d, cand, strip, model, image, weight, psf, partials,  \
+            lensed_conv_sweep_item<PW_, PH_, OUT>(d, cand, strip, seg, model, image, weight, psf, partials,  \
                                                   conv_out, chi2_out, trace, dark, lrow);               \
             return;                                                                                     \
         }                                                                                               \
