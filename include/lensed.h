@@ -253,7 +253,7 @@ typedef struct {
     double list_fraction; /* the render walks the cull's list of lit 4 x 4 quads while under this fraction
                              of all quads is lit, else every item, skipping dark squares by their flag
                              (0.75; negative: never the list, above 1: always) */
-    double render_grid;   /* render blocks as a multiple of the resident count (1) */
+    double render_grid;   /* render blocks as a multiple of the resident count (16; 4 after a cull pass) */
     double cull_grid;     /* pixel-cull blocks, the same (4) */
     double conv_grid;     /* convolution blocks, the same (1) */
     int conv_rows;        /* output rows per thread of the convolution tile (4 rows of threads): 2, 8 or 16

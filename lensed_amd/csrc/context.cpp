@@ -431,7 +431,15 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         return -1;
     }
     // persistent grids sized by what stays resident with this launch's LDS,
-    // times the requested multiples
+    // times the requested multiples.  The render's default is 16 times over
+    // the items and 4 times over the cull's list: with as many blocks as are
+    // resident, whole rounds of equal work leave the last one part empty
+    // (12544 items on 2048 blocks: 7 rounds for 6.1), while further blocks
+    // start as others end.  256 candidates of 100 x 100 (SIE + Sersic): 698 us
+    // at 1, 670 at 4, 604 at 16; 512 of 512 x 512 (table): 12.7, 11.7, 11.6
+    // ms; the list's blocks lose more to starting than they gain beyond 4
+    // (512 of 256 x 256, series: 665, 612, 635 us).
+    const double default_render_grid = L.any_cull ? 4.0 : 16.0;
     {
         auto scaled = [&](int resident, double m) {
             return std::max(1, (int)std::lround(resident * (m > 0 ? m : 1.0)));
@@ -443,7 +451,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         if (sweep) L.grid_conv = (ic + 3) / 4;  // not persistent: four strips per block, every strip its wave
         nb = 0;
         hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, l->f_render, LENSED_RENDER_BS, L.lds_render);
-        L.grid_render = scaled(std::max(1, nb) * l->cu_count, tq.render_grid);
+        L.grid_render = scaled(std::max(1, nb) * l->cu_count, tq.render_grid > 0 ? tq.render_grid : default_render_grid);
         // the cull's blocks take a few items each by default (its items differ in cost by
         // their unsettled squares; 4x evens the tail: C3 cull 0.18 -> 0.14 ms)
         L.grid_cull = scaled(std::max(1, nb) * l->cu_count, tq.cull_grid > 0 ? tq.cull_grid : 4.0);
@@ -456,7 +464,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         L.list_max = f < 0 ? 0 : f > 1 ? INT_MAX : (int)std::min<double>(INT_MAX, std::ceil(f * quads));
         L.tune.list_fraction = f;
     }
-    L.tune.render_grid = tq.render_grid > 0 ? tq.render_grid : 1.0;
+    L.tune.render_grid = tq.render_grid > 0 ? tq.render_grid : default_render_grid;
     L.tune.cull_grid = tq.cull_grid > 0 ? tq.cull_grid : 4.0;
     L.tune.conv_grid = tq.conv_grid > 0 ? tq.conv_grid : 1.0;
     L.tune.conv_rows = L.conv_rows;
@@ -680,7 +688,7 @@ static int run_layout(::lensed* l, Layout& L) {
 // layout's systems and candidate counts
 static std::string tune_key(const ::lensed* l, const std::vector<size_t>& ncand, bool emulate) {
     std::ostringstream k;
-    k << "lensed-tune-2 " << device_arch(l->device) << " cu" << l->cu_count << " prog" << std::hex
+    k << "lensed-tune-3 " << device_arch(l->device) << " cu" << l->cu_count << " prog" << std::hex
       << fnv1a(l->source) << " cc" << fnv1a(compiler_identity()) << std::dec << " emu" << (emulate ? 1 : 0) << " flags" << (l->flags & ~(LENSED_PROFILE | LENSED_GRAPH));
     for (size_t s = 0; s < l->sys.size(); ++s)
         k << " " << l->sys[s].width << "x" << l->sys[s].height << "p" << l->sys[s].psfw << "x" << l->sys[s].psfh
@@ -984,6 +992,7 @@ lensed* lensed_create(const lensed_system* systems, size_t nsys, const lensed_op
         l->sys.push_back(S);
     }
     if (psf.empty()) psf.push_back(0.0f);
+    for (const auto& m : models) l->block_pad = std::max(l->block_pad, model_data_words(m));
 
     std::vector<PsfShape> shapes;
     for (const auto& S : l->sys) {
@@ -1084,7 +1093,7 @@ lensed* lensed_create(const lensed_system* systems, size_t nsys, const lensed_op
         hipMalloc(&l->d_psf, psf.size() * 4) != hipSuccess ||
         hipMalloc(&l->d_quad, quad.size() * 4) != hipSuccess ||
         hipMalloc(&l->d_params, std::max<size_t>(1, l->cap_params) * 4) != hipSuccess ||
-        hipMalloc(&l->d_blocks, (l->cap_blocks + 256) * 4) != hipSuccess ||
+        hipMalloc(&l->d_blocks, (l->cap_blocks + l->block_pad) * 4) != hipSuccess ||
         hipMalloc(&l->d_model, l->cap_model * 4) != hipSuccess ||
         hipMalloc(&l->d_err, maxpix * 4) != hipSuccess || hipMalloc(&l->d_conv, maxpix * 4) != hipSuccess ||
         hipMalloc(&l->d_chi2, maxpix * 4) != hipSuccess ||
@@ -1508,7 +1517,7 @@ int lensed_loglike_batch_noalloc(lensed* l, size_t s, const double* cubes, size_
     const size_t squares = nc * (size_t)d.ntile_r * (LENSED_RENDER_BS / 64);
     const size_t sizes[] = {sizeof(lensed_desc),
                             nc * d.npar * 4,
-                            (nc * d.dwords + 256) * 4,
+                            (nc * d.dwords + l->block_pad) * 4,
                             d.table_mode || S.cull ? nc * LENSED_NPRE_STRIDE(d.table_mode ? d.nq : 0) * 16 : 16,
                             d.table_mode ? nc * LENSED_EPL_TABLE_F4 * 16 : 16,
                             nc * (size_t)d.npix * 4,

@@ -164,6 +164,7 @@ struct lensed {
     // pinned host staging
     float* h_params = nullptr;
     double* h_logl = nullptr;
+    size_t block_pad = 4;  // words past the object blocks: every load takes a whole LENSED_DWORDS block
     size_t cap_params = 0, cap_blocks = 0, cap_model = 0, cap_partials = 0, cap_out = 0, cap_tables = 0;
     std::map<std::vector<size_t>, lsd::Layout> layouts;
     std::string source;          // generated program (for dumps)

@@ -121,7 +121,7 @@ int autotune(const TuneTimer& timer, bool culls, lensed_tuning* best) {
             c.list_fraction = lf;
             if (try_render(c)) return -1;
         }
-    for (double g : {0.5, 2.0, 4.0}) {
+    for (double g : {1.0, 4.0, 8.0, 16.0}) {  // (the default is 16, 4 with a list)
         lensed_tuning c = cur;
         c.render_grid = g;
         if (try_render(c)) return -1;

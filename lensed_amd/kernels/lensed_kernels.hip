@@ -144,6 +144,9 @@ __device__ inline bool lensed_render_pixel(const lensed_desc& d, int tile, int w
 // loop runs in the thread with the node table in scalar registers and the
 // candidate's object block held in SGPRs (wave-uniform), so the per-ray work
 // is pure VALU.
+// (The block is read whole, LENSED_DWORDS words, in a few wide scalar loads;
+// the words past a smaller model's own are not used, and the host keeps that
+// much room after the last block.)
 template <int K, bool ERR>
 __device__ inline void lensed_render_item(const lensed_desc& d, int cand, int px, int py, bool on, bool restage,
                                           const u32* __restrict__ blocks, const float4* __restrict__ quad,
@@ -153,7 +156,7 @@ __device__ inline void lensed_render_item(const lensed_desc& d, int cand, int px
     u32 blk[LENSED_DWORDS];
     const u32* gb = blocks + d.block_off + (long long)cand * d.dwords;
 #pragma unroll
-    for (int i = 0; i < LENSED_DWORDS; ++i) blk[i] = i < d.dwords ? __builtin_amdgcn_readfirstlane(gb[i]) : 0u;
+    for (int i = 0; i < LENSED_DWORDS; ++i) blk[i] = __builtin_amdgcn_readfirstlane(gb[i]);
     const float4* q = quad + d.quad_off;
     if (d.table_mode && restage) {  // the candidate's EPL angular table, staged in LDS
         __syncthreads();  // the previous candidate's table is no longer read
@@ -228,8 +231,8 @@ extern "C" __global__ __launch_bounds__(LENSED_RENDER_BS) __attribute__((amdgpu_
         }
         int s = lensed_find_sys<0>(sys, nsys, item);
         const lensed_desc& d = sys[s];
-        int local = item - d.item_r;
-        int cand = local / d.ntile_r;
+        // (uniform, and known so: what is indexed by it stays scalar)
+        const int cand = __builtin_amdgcn_readfirstlane((item - d.item_r) / d.ntile_r);
         int px = 0, py = 0;
         bool on;
         if (listed) {
@@ -303,7 +306,7 @@ __device__ inline int lensed_cull_wave(const lensed_desc& d, int cand, int g0, i
     u32 blk[LENSED_DWORDS];
     const u32* gb = blocks + d.block_off + (long long)cand * d.dwords;
 #pragma unroll
-    for (int i = 0; i < LENSED_DWORDS; ++i) blk[i] = i < d.dwords ? __builtin_amdgcn_readfirstlane(gb[i]) : 0u;
+    for (int i = 0; i < LENSED_DWORDS; ++i) blk[i] = __builtin_amdgcn_readfirstlane(gb[i]);
     const int pairs = d.table_mode ? d.nq : 0;
     const float4* ccg = npre + d.npre_off + (long long)cand * LENSED_NPRE_STRIDE(pairs) + pairs;
     lcl::float4 cc[LENSED_NPRE_CULL];
