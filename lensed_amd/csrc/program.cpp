@@ -347,6 +347,15 @@ static bool slope_culls(const std::vector<ModelObject>& objs) {
     return true;
 }
 
+bool model_holds(const std::vector<ModelObject>& objs) {
+    // at most 64 words, so that the loop stays within its 128 registers; not
+    // with an EPL series per ray (lensed_render_item has both sides measured)
+    if (model_data_words(objs) > 64) return false;
+    for (const auto& ob : objs)
+        if (ob.type == OBJ_LENS && !ob.table && object_tabulates(ob.name)) return false;
+    return true;
+}
+
 bool model_culls(const std::vector<ModelObject>& objs) { return frame_culls(objs) || slope_culls(objs); }
 
 std::string compute_function(const std::vector<ModelObject>& objs, int k) {
@@ -402,9 +411,14 @@ std::string compute_function(const std::vector<ModelObject>& objs, int k) {
     // of the deflection is subtracted from it.  The guard then sees the
     // deflection without the shear, which is finite wherever the shear is
     // (finite parameters), so the rays it rejects are the same.
+    // A rejected ray goes to -1e10 itself instead of to that distance from
+    // where it was (the same number in FP32 within 512 pixels of the origin,
+    // 1024 pixels apart at most steps further out, and no source's light
+    // either way): the subtraction then stands between the comparison and the
+    // selects that wait for it.
     auto close_plane = [&]() {
-        o << "        y = " << (lin ? "float2(pre.z, pre.w)" : "y")
-          << " - (lensed_deflection_ok(a) ? a : float2(1E10f, 1E10f));\n    }\n";
+        o << "        const float2 r = " << (lin ? "float2(pre.z, pre.w)" : "y") << " - a;\n"
+          << "        y = lensed_deflection_ok(a) ? r : float2(-1E10f, -1E10f);\n    }\n";
         plane_open = false;
     };
     for (size_t i = 0; i < objs.size(); ++i) {

@@ -141,9 +141,16 @@ __device__ inline bool lensed_render_pixel(const lensed_desc& d, int tile, int w
 }
 
 // One thread per pixel (px, py; on: the thread has one); the 2-D quadrature
-// loop runs in the thread with the node table in scalar registers and the
-// candidate's object block held in SGPRs (wave-uniform), so the per-ray work
-// is pure VALU.
+// loop runs in the thread with the node table in scalar registers.  The
+// candidate's object block is wave-uniform and comes in by scalar loads; for
+// most models it is then held in vector registers (model_holds): multiplies,
+// adds and FMAs of vector registers and literals issue at up to 1.75 per CU
+// and cycle, those with a scalar operand at 0.93.  Measured over the ray
+// loops, cycles of a CU per wave and ray, scalar and vector: SIE + Sersic 202
+// and 182, SIE + shear + two sources + sky 203 and 183, tabulated EPL + two
+// Sersic + sky 73.7 and 70.2, tabulated EPL + Gaussian 41.5 and 39.2.  The EPL
+// series, which takes a coefficient per Horner step and is half fast
+// instructions either way, loses: 81.5 and 84 (not held).
 // (The block is read whole, LENSED_DWORDS words, in a few wide scalar loads;
 // the words past a smaller model's own are not used, and the host keeps that
 // much room after the last block.)
@@ -157,6 +164,10 @@ __device__ inline void lensed_render_item(const lensed_desc& d, int cand, int px
     const u32* gb = blocks + d.block_off + (long long)cand * d.dwords;
 #pragma unroll
     for (int i = 0; i < LENSED_DWORDS; ++i) blk[i] = __builtin_amdgcn_readfirstlane(gb[i]);
+    if constexpr (lcl::model_holds(K)) {
+#pragma unroll
+        for (int i = 0; i < LENSED_DWORDS; ++i) asm("" : "+v"(blk[i]));
+    }
     const float4* q = quad + d.quad_off;
     if (d.table_mode && restage) {  // the candidate's EPL angular table, staged in LDS
         __syncthreads();  // the previous candidate's table is no longer read
@@ -175,6 +186,7 @@ __device__ inline void lensed_render_item(const lensed_desc& d, int cand, int px
             // pixel's part and the node's (from set_params, scalar loads)
             const lcl::float4 base = lcl::epl_pre_model<K>(blk, lcl::float2(cx, cy), true);
             const float4* np_c = npre + d.npre_off + (long long)cand * LENSED_NPRE_STRIDE(d.nq);
+
             for (int n = 0; n < d.nq; ++n) {
                 const float4 node = q[n];
                 const float4 np = np_c[n];
@@ -185,6 +197,7 @@ __device__ inline void lensed_render_item(const lensed_desc& d, int cand, int px
                 if (ERR) e += node.w * v;
             }
         } else {
+
             for (int n = 0; n < d.nq; ++n) {
                 const float4 node = q[n];
                 float v = lcl::compute_model<K>(blk, lcl::float2(cx + node.x, cy + node.y), nullptr,
@@ -199,9 +212,10 @@ __device__ inline void lensed_render_item(const lensed_desc& d, int cand, int px
     }
 }
 
-// eight waves per SIMD (at most 64 VGPRs): the ray loop's latencies
-// (transcendentals, LDS lookups) are hidden by the other waves
-extern "C" __global__ __launch_bounds__(LENSED_RENDER_BS) __attribute__((amdgpu_waves_per_eu(8, 8))) void lensed_render(
+// four to eight waves per SIMD (at most 128 VGPRs, about 65 with the block
+// held): two already keep the vector pipes three quarters full, and a limit
+// of 64 VGPRs costs the two-source models 13 % in copies
+extern "C" __global__ __launch_bounds__(LENSED_RENDER_BS) __attribute__((amdgpu_waves_per_eu(4, 8))) void lensed_render(
     const lensed_desc* __restrict__ sys, int nsys, int nitems,
     const u32* __restrict__ blocks, const float4* __restrict__ quad, const float4* __restrict__ tables,
     const float4* __restrict__ npre, const int* __restrict__ live, const int* __restrict__ trace,

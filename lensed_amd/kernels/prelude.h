@@ -202,6 +202,14 @@ inline float2 max(float2 a, float2 b) { return float2(max(a.x, b.x), max(a.y, b.
 inline float2 min(float2 a, float b) { return float2(min(a.x, b), min(a.y, b)); }
 inline float2 max(float2 a, float b) { return float2(max(a.x, b), max(a.y, b)); }
 
+// Marks a branch as one to jump around: code that most candidates do without,
+// where the compiler would rather do it for all and select.
+inline void lensed_branch() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("");
+#endif
+}
+
 // ---------------------------------------------------------------- geometry
 inline float dot(float2 a, float2 b) { return a.x * b.x + a.y * b.y; }
 inline float dot(float4 a, float4 b) { return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w; }

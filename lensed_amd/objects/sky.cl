@@ -17,7 +17,15 @@ data
 
 static float foreground(local data* this, float2 x)
 {
-    return this->level + dot(this->grad, x - (float2)(1, 1));
+    float f = this->level;
+    // (no gradient, the default: the same value without seven of a ray's
+    // instructions, of 66 behind a tabulated lens with two Sersic sources)
+    if(this->grad.x != 0 || this->grad.y != 0)
+    {
+        lensed_branch();
+        f += dot(this->grad, x - (float2)(1, 1));
+    }
+    return f;
 }
 
 static void set(local data* this, float bg, float dx, float dy)
