@@ -293,16 +293,26 @@ static void evict_layouts(::lensed* l) {
 // everything of a launch layout but its device descriptors (no allocation
 // on the device); 0 on success
 static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L) {
-    // conv tile height: the tall tiles unless the launch would leave CUs idle
-    long long tall_items = 0;
-    for (size_t s = 0; s < l->sys.size(); ++s) {
-        const System& S = l->sys[s];
-        tall_items += (long long)ncand[s] * ((S.width + LENSED_CONV_TX - 1) / LENSED_CONV_TX) *
-                      ((S.height + LENSED_CONV_TY * LENSED_CONV_RY - 1) / (LENSED_CONV_TY * LENSED_CONV_RY));
-    }
-    L.conv_small = tall_items < 2LL * l->cu_count;
+    // conv tile height: the tallest of which the launch has two per CU.  (us,
+    // 8-, 32- and 64-row tiles, by the number of 64-row ones: direct 31 x 31
+    // taps 256: 46, 41, 47; 512: 84, 66, 52; 32768: 4782, 3782, 2750; two
+    // passes of 21 taps 256: 12, 11, 12; 512: 18, 13.0, 13.6; 1024: 30, 17.5,
+    // 16.7; 16384: 366, 204, 177)
+    auto tiles = [&](int rows) {
+        long long n = 0;
+        for (size_t s = 0; s < l->sys.size(); ++s) {
+            const System& S = l->sys[s];
+            n += (long long)ncand[s] * ((S.width + LENSED_CONV_TX - 1) / LENSED_CONV_TX) *
+                 ((S.height + LENSED_CONV_TY * rows - 1) / (LENSED_CONV_TY * rows));
+        }
+        return n;
+    };
+    L.conv_small = tiles(LENSED_CONV_RY) < 2LL * l->cu_count;
     const lensed_tuning& tq = l->tune_req;
-    L.conv_rows = tq.conv_rows ? tq.conv_rows : (L.conv_small ? LENSED_CONV_RY_SMALL : LENSED_CONV_RY);
+    const int rows_default = L.conv_small                                       ? LENSED_CONV_RY_SMALL
+                             : tiles(LENSED_CONV_RY_TALL) < 2LL * l->cu_count ? LENSED_CONV_RY
+                                                                              : LENSED_CONV_RY_TALL;
+    L.conv_rows = tq.conv_rows ? tq.conv_rows : rows_default;
     // the column sweep: every system with candidates has a rank-1 separable
     // PSF of at most 21 x 21, and at most 512 rows.  It is the default
     // where every such system is also culled: it skips the rows the cull
@@ -329,7 +339,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
     }
     if (!tq.conv_rows && sweep_ok && all_culled && strips >= 2LL * l->cu_count) L.conv_rows = LENSED_CONV_SWEEP;
     if (L.conv_rows == LENSED_CONV_SWEEP && !sweep_ok)
-        L.conv_rows = L.conv_small ? LENSED_CONV_RY_SMALL : LENSED_CONV_RY;
+        L.conv_rows = rows_default;
     if (L.conv_rows == LENSED_CONV_RY_TALL) {
         // the 64-row tile only where its LDS stays within 64 KiB
         for (size_t s = 0; s < l->sys.size(); ++s) {

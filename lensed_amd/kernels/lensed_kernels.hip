@@ -788,6 +788,17 @@ __device__ inline void lensed_conv_generic(const lensed_desc& d, const float* __
     }
 }
 
+// A PSF tap of the 64-row tile, held in a vector register: FMAs of vector
+// registers issue at up to 1.75 per CU and cycle, with a scalar operand at
+// 0.93, and a tap serves sixteen of them there.  (The shorter tiles keep
+// theirs scalar: with half the FMAs a tap the moves and the registers, six
+// waves' worth, outweigh it.)
+template <bool HOLD>
+__device__ inline float lensed_tap(float w) {
+    if (HOLD) asm("" : "+v"(w));
+    return w;
+}
+
 // PSF size fixed at compile time: taps unrolled into scalar registers and
 // every LDS value reused from VGPRs.  Separable: the row pass computes four
 // adjacent outputs per thread from one vector read of 4 + PW - 1 values;
@@ -807,7 +818,9 @@ __device__ inline void lensed_conv_sep_rank(const float* __restrict__ cf, float*
     constexpr int NX = 4, NV = (NX + PW - 1 + 3) / 4;
     constexpr int TS = TMP_IN_TILE ? STRIDE : TX;
     float* tmp = TMP_IN_TILE ? tile : tile + STRIDE * CH;
-    const float* rf = cf + PH;
+    float rf[PW], cv[PH];
+#pragma unroll
+    for (int i = 0; i < PW; ++i) rf[i] = lensed_tap<RY == LENSED_CONV_RY_TALL>(cf[PH + i]);
     for (int r = threadIdx.x / (TX / NX); r < CH; r += BS / (TX / NX)) {
         const int x0 = (threadIdx.x % (TX / NX)) * NX;
         const float4* src = (const float4*)(tile + r * STRIDE + x0);
@@ -831,12 +844,16 @@ __device__ inline void lensed_conv_sep_rank(const float* __restrict__ cf, float*
     }
     __syncthreads();
     float col[NC];
+    // (a column of more than 21 taps beside its RY + PH - 1 values leaves no
+    // registers for them)
+#pragma unroll
+    for (int j = 0; j < PH; ++j) cv[j] = lensed_tap<RY == LENSED_CONV_RY_TALL && PH <= 21>(cf[j]);
 #pragma unroll
     for (int q = 0; q < NC; ++q) col[q] = tmp[(ly * RY + q) * TS + lx];
 #pragma unroll
     for (int j = 0; j < PH; ++j)
 #pragma unroll
-        for (int r = 0; r < RY; ++r) acc[r] = __builtin_fmaf(cf[j], col[r + PH - 1 - j], acc[r]);
+        for (int r = 0; r < RY; ++r) acc[r] = __builtin_fmaf(cv[j], col[r + PH - 1 - j], acc[r]);
     __syncthreads();
 }
 
@@ -857,13 +874,15 @@ __device__ inline void lensed_conv_fixed(const lensed_desc& d, const float* __re
         const float* pt = psf + d.psft_off;  // [PW][PH]
 #pragma unroll 1
         for (int i = 0; i < PW; ++i) {
-            float col[NC];
+            float col[NC], tap[PH];
+#pragma unroll
+            for (int j = 0; j < PH; ++j) tap[j] = lensed_tap<RY == LENSED_CONV_RY_TALL>(pt[i * PH + j]);
 #pragma unroll
             for (int q = 0; q < NC; ++q) col[q] = tile[(ly * RY + q) * STRIDE + lx + PW - 1 - i];
 #pragma unroll
             for (int j = 0; j < PH; ++j)
 #pragma unroll
-                for (int r = 0; r < RY; ++r) acc[r] += pt[i * PH + j] * col[r + PH - 1 - j];
+                for (int r = 0; r < RY; ++r) acc[r] += tap[j] * col[r + PH - 1 - j];
         }
         __syncthreads();
     }
