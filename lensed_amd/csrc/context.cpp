@@ -313,6 +313,17 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
                              : tiles(LENSED_CONV_RY_TALL) < 2LL * l->cu_count ? LENSED_CONV_RY
                                                                               : LENSED_CONV_RY_TALL;
     L.conv_rows = tq.conv_rows ? tq.conv_rows : rows_default;
+    long long squares = 0;  // 64 pixels each: a wave of the render
+    bool tables = false;
+    for (size_t s = 0; s < l->sys.size(); ++s) {
+        squares += 4LL * (long long)ncand[s] * l->sys[s].ntile_r;
+        tables = tables || (ncand[s] && l->sys[s].table);
+    }
+    // no cull pass where tracing every ray takes no longer than finding the
+    // dark ones (us of cull and render, with and without the pass, 256 x 256:
+    // table 1 candidate 27, 16; 4: 29, 23; 8: 33, 35; series 1: 26, 16; 2: 27,
+    // 24; 4: 31, 40)
+    const bool no_cull = (l->flags & LENSED_NO_CULL) || squares < (tables ? 8LL : 3LL) * 4 * l->cu_count;
     // the column sweep: every system with candidates has a rank-1 separable
     // PSF of at most 21 x 21, and at most 512 rows.  It is the default
     // where every such system is also culled: it skips the rows the cull
@@ -335,7 +346,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         if (!S.psfw || S.sep_rank != 1 || S.psfw > LENSED_SWEEP_MAX_PSF || S.psfh > LENSED_SWEEP_MAX_PSF ||
             S.height > LENSED_SWEEP_MAX_H)
             sweep_ok = false;
-        if (!S.cull || (l->flags & LENSED_NO_CULL)) all_culled = false;
+        if (!S.cull || no_cull) all_culled = false;
     }
     if (!tq.conv_rows && sweep_ok && all_culled && strips >= 2LL * l->cu_count) L.conv_rows = LENSED_CONV_SWEEP;
     if (L.conv_rows == LENSED_CONV_SWEEP && !sweep_ok)
@@ -408,7 +419,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         d.psft_off = S.psft_off;
         d.npre_off = npre_off;
         d.qrad = S.qrad;
-        d.cull = S.cull && !(l->flags & LENSED_NO_CULL) ? 1 : 0;
+        d.cull = S.cull && !no_cull ? 1 : 0;
         d.dark_off = S.dark_off;
         d.sweep_seg = seg;
         L.any_cull = L.any_cull || d.cull;
@@ -471,6 +482,20 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         L.grid_cull = scaled(std::max(1, nb) * l->cu_count, tq.cull_grid > 0 ? tq.cull_grid : 4.0);
     }
     L.conv_order = tq.conv_order == 2 ? 1 : 0;
+    {
+        // a block per 64 pixels, their rays shared among its waves, where the
+        // launch has too few pixels for a wave to trace its own (us of render,
+        // a wave per 64 pixels and shared: SIE + Sersic 196 squares 46, 13;
+        // 1568: 37, 34; 6272: 105, 103; series 1024: 20, 16; 4096: 39, 41;
+        // table 1024: 18, 13; 2048: 17, 19, each block staging the table;
+        // culled, most of the squares dark: 8192: 49, 33; 16384: 45, 40;
+        // 32768: 57, 62)
+        const long long per = L.any_cull ? 16 : tables ? 1 : 3;
+        int nqmax = 0;
+        for (const auto& d : L.desc) nqmax = std::max(nqmax, d.nq);
+        L.lds_wide = L.lds_render + (size_t)nqmax * 64 * sizeof(float);
+        L.wide = squares <= per * 4 * l->cu_count && nqmax > 4 && L.lds_wide <= 65536;
+    }
     {
         // the render walks the list while under list_fraction of the quads are lit
         const double f = tq.list_fraction == 0 ? 0.75 : tq.list_fraction;
@@ -632,10 +657,12 @@ static int enqueue_chain(::lensed* l, Layout& L, const Buffers& B, bool prof, fl
         rec(9);
     }
     {
-        int grid = std::min(L.n_render, L.grid_render);
+        int grid = std::min(L.n_render, L.grid_render), table_f4 = (int)(L.lds_render / 16);
         void* a[] = {&desc,  &nsys,  &L.n_render, &blocks,    &l->d_quad,  &tables,
-                     &npre,  &live,  &trace,      &model,     &err_plane,  &L.list_max};
-        if (launch(l->f_render, grid, LENSED_RENDER_BS, L.lds_render, st, a)) return -1;
+                     &npre,  &live,  &trace,      &model,     &err_plane,  &L.list_max, &table_f4};
+        if (L.wide) grid = std::min(4 * L.n_render, L.grid_render);
+        if (launch(L.wide ? l->f_wide : l->f_render, grid, LENSED_RENDER_BS, L.wide ? L.lds_wide : L.lds_render, st, a))
+            return -1;
     }
     rec(4);
     {
@@ -1050,6 +1077,7 @@ lensed* lensed_create(const lensed_system* systems, size_t nsys, const lensed_op
         hipModuleGetFunction(&l->f_tables, l->module, "lensed_epl_tables") != hipSuccess ||
         hipModuleGetFunction(&l->f_set_tables, l->module, "lensed_set_params_tables") != hipSuccess ||
         hipModuleGetFunction(&l->f_dark, l->module, "lensed_dark_partials") != hipSuccess ||
+        hipModuleGetFunction(&l->f_wide, l->module, "lensed_render_wide") != hipSuccess ||
         hipModuleGetFunction(&l->f_cull, l->module, "lensed_cull") != hipSuccess ||
         hipModuleGetFunction(&l->f_conv_tall, l->module, "lensed_conv_chi2_tall") != hipSuccess ||
         hipModuleGetFunction(&l->f_conv_sweep, l->module, "lensed_conv_chi2_sweep") != hipSuccess ||

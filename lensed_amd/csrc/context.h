@@ -81,6 +81,8 @@ struct Layout {
     bool any_cull = false;          // some system culls pixels before the render (lensed_cull)
     int grid_conv = 0, grid_render = 0;  // resident blocks for this launch's LDS use
     int grid_cull = 0;
+    bool wide = false;              // the render shares each pixel's rays among waves (lensed_render_wide)
+    size_t lds_wide = 0;
     int list_max = 0;               // the render walks the cull's list below this many lit quads
     int conv_rows = 8;              // rows per thread of the convolution tile (2, 8, 16)
     int conv_order = 0;             // convolution item order (kernel argument, 0 or 1)
@@ -126,7 +128,7 @@ struct lensed {
     hipModule_t module = nullptr;
     hipFunction_t f_set = nullptr, f_render = nullptr, f_conv = nullptr, f_conv_small = nullptr, f_final = nullptr,
                   f_tables = nullptr, f_cull = nullptr, f_conv_tall = nullptr, f_conv_sweep = nullptr,
-                  f_conv_sweep_out = nullptr, f_set_tables = nullptr, f_dark = nullptr;
+                  f_conv_sweep_out = nullptr, f_set_tables = nullptr, f_dark = nullptr, f_wide = nullptr;
     lensed_tuning tune_req{};    // requested launch shapes (zero fields: defaults)
     int cu_count = 1;
     hipStream_t stream = nullptr;

@@ -140,6 +140,17 @@ __device__ inline bool lensed_render_pixel(const lensed_desc& d, int tile, int w
     return px < d.width && py < d.height;
 }
 
+// Pixel (lane % 16) of quad q % 4 of square (q / 4) % 4 of render item q / 16,
+// as the render list holds quads; false outside the image and for a pad (-1).
+__device__ inline bool lensed_list_pixel(const lensed_desc& d, int cand, int q, int lane, int& px, int& py) {
+    const int ntx = (d.width + LENSED_RENDER_SIDE - 1) / LENSED_RENDER_SIDE;
+    const int tile = (q >> 4) - d.item_r - cand * d.ntile_r, by = tile / ntx, bx = tile - by * ntx;
+    const int w = (q >> 2) & 3, p = lane & 15;
+    px = bx * LENSED_RENDER_SIDE + (w & 1) * 8 + (q & 1) * 4 + (p & 3);
+    py = by * LENSED_RENDER_SIDE + (w >> 1) * 8 + ((q >> 1) & 1) * 4 + (p >> 2);
+    return q >= 0 && px < d.width && py < d.height;
+}
+
 // One thread per pixel (px, py; on: the thread has one); the 2-D quadrature
 // loop runs in the thread with the node table in scalar registers.  The
 // candidate's object block is wave-uniform and comes in by scalar loads; for
@@ -250,13 +261,7 @@ extern "C" __global__ __launch_bounds__(LENSED_RENDER_BS) __attribute__((amdgpu_
         int px = 0, py = 0;
         bool on;
         if (listed) {
-            // pixel (lane % 16) of quad q % 4 of square (q / 4) % 4 of render item q / 16
-            const int ntx = (d.width + LENSED_RENDER_SIDE - 1) / LENSED_RENDER_SIDE;
-            const int tile = (q >> 4) - d.item_r - cand * d.ntile_r, by = tile / ntx, bx = tile - by * ntx;
-            const int w = (q >> 2) & 3, p = lane & 15;
-            px = bx * LENSED_RENDER_SIDE + (w & 1) * 8 + (q & 1) * 4 + (p & 3);
-            py = by * LENSED_RENDER_SIDE + (w >> 1) * 8 + ((q >> 1) & 1) * 4 + (p >> 2);
-            on = q >= 0 && px < d.width && py < d.height;
+            on = lensed_list_pixel(d, cand, q, lane, px, py);
         } else {
             on = true;
             if (live && d.cull)  // flags exist for the culled systems' squares only
@@ -278,6 +283,126 @@ extern "C" __global__ __launch_bounds__(LENSED_RENDER_BS) __attribute__((amdgpu_
         break;
             LENSED_FOR_MODELS(LENSED_RENDER_CASE)
 #undef LENSED_RENDER_CASE
+            default: break;
+        }
+    }
+}
+
+// The render of a launch too small to fill the device: a block per 64 pixels
+// (a square of the walk, or four quads of the list), its waves sharing the
+// rays of the pixels by node.  A wave of lensed_render traces its pixels' rays
+// one after the other, so one candidate's image takes the latency of 49 rays
+// in a row on a few waves.  Here each ray's value goes to LDS and
+// the first wave adds them up in node order with the same operations as
+// lensed_render, so the bits are the same.
+template <int K, bool ERR>
+__device__ inline void lensed_render_wide_item(const lensed_desc& d, int cand, int px, int py, bool on, bool restage,
+                                               const u32* __restrict__ blocks, const float4* __restrict__ quad,
+                                               const float4* __restrict__ tables, const float4* __restrict__ npre,
+                                               float4* tab_lds, float* rays, float* __restrict__ model,
+                                               float* __restrict__ errp)
+{
+    u32 blk[LENSED_DWORDS];
+    const u32* gb = blocks + d.block_off + (long long)cand * d.dwords;
+#pragma unroll
+    for (int i = 0; i < LENSED_DWORDS; ++i) blk[i] = __builtin_amdgcn_readfirstlane(gb[i]);
+    if constexpr (lcl::model_holds(K)) {
+#pragma unroll
+        for (int i = 0; i < LENSED_DWORDS; ++i) asm("" : "+v"(blk[i]));
+    }
+    const float4* q = quad + d.quad_off;
+    if (d.table_mode && restage) {
+        const float4* src = tables + d.table_off + (long long)cand * LENSED_EPL_TABLE_F4;
+        for (int i = threadIdx.x; i < LENSED_EPL_TABLE_F4; i += LENSED_RENDER_BS) tab_lds[i] = src[i];
+        __syncthreads();
+    }
+    constexpr int waves = LENSED_RENDER_BS / 64;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int lane = (int)threadIdx.x & 63;
+    const int n0 = d.nq * wave / waves, n1 = d.nq * (wave + 1) / waves;
+    if (on) {
+        const float cx = d.pcs[0] + d.pcs[2] * (float)px;
+        const float cy = d.pcs[1] + d.pcs[3] * (float)py;
+        if (d.table_mode) {
+            const lcl::float4 base = lcl::epl_pre_model<K>(blk, lcl::float2(cx, cy), true);
+            const float4* np_c = npre + d.npre_off + (long long)cand * LENSED_NPRE_STRIDE(d.nq);
+            for (int n = n0; n < n1; ++n) {
+                const float4 node = q[n];
+                const float4 np = np_c[n];
+                const lcl::float4 pre(base.x + np.x, base.y + np.y, base.z + np.z, base.w + np.w);
+                rays[n * 64 + lane] = lcl::compute_model<K>(blk, lcl::float2(cx + node.x, cy + node.y),
+                                                            (const lcl::float4*)tab_lds, pre);
+            }
+        } else {
+            for (int n = n0; n < n1; ++n) {
+                const float4 node = q[n];
+                rays[n * 64 + lane] = lcl::compute_model<K>(blk, lcl::float2(cx + node.x, cy + node.y), nullptr,
+                                                            lcl::float4(0.0f, 0.0f, 0.0f, 0.0f));
+            }
+        }
+    }
+    __syncthreads();
+    if (wave == 0 && on) {
+        float f = 0.0f, e = 0.0f;
+        for (int n = 0; n < d.nq; ++n) {
+            const float4 node = q[n];
+            const float v = rays[n * 64 + lane];
+            f = __builtin_fmaf(node.z, v, f);
+            if (ERR) e = __builtin_fmaf(node.w, v, e);
+        }
+        const long long o = d.model_off + (long long)cand * d.npix + py * d.width + px;
+        model[o] = f;
+        if (ERR) errp[o] = e;
+    }
+    __syncthreads();  // the next unit writes the rays again
+}
+
+extern "C" __global__ __launch_bounds__(LENSED_RENDER_BS) __attribute__((amdgpu_waves_per_eu(4, 8))) void lensed_render_wide(
+    const lensed_desc* __restrict__ sys, int nsys, int nitems,
+    const u32* __restrict__ blocks, const float4* __restrict__ quad, const float4* __restrict__ tables,
+    const float4* __restrict__ npre, const int* __restrict__ live, const int* __restrict__ trace,
+    float* __restrict__ model, float* __restrict__ errp, int list_max, int table_f4)
+{
+    extern __shared__ float4 tab_lds[];
+    float* rays = (float*)(tab_lds + table_f4);
+    const int lane = (int)threadIdx.x & 63;
+    const bool listed = live && live[0] < list_max;
+    const int units = listed ? live[0] / 4 : nitems * 4;
+    int staged = -1;
+    for (int u = (int)blockIdx.x; u < units; u += (int)gridDim.x) {
+        int item = u >> 2, q = -1;
+        if (listed) {
+            const int* e = live + 1;
+            if (e[4 * u] < 0) continue;  // the whole quarter is padding
+            item = e[4 * u] >> 4;
+            q = e[4 * u + (lane >> 4)];
+        }
+        const int s = lensed_find_sys<0>(sys, nsys, item);
+        const lensed_desc& d = sys[s];
+        const int cand = __builtin_amdgcn_readfirstlane((item - d.item_r) / d.ntile_r);
+        int px = 0, py = 0;
+        bool on;
+        if (listed) {
+            on = lensed_list_pixel(d, cand, q, lane, px, py);
+        } else {
+            if (live && d.cull && trace[u] == 0) continue;  // a culled system's dark square
+            on = lensed_render_pixel(d, item - d.item_r - cand * d.ntile_r, u & 3, px, py);
+        }
+        const int key = d.item_r + cand * d.ntile_r;  // block-uniform
+        const bool restage = key != staged;
+        staged = key;
+        switch (d.model) {
+#define LENSED_WIDE_CASE(K)                                                                                     \
+    case K:                                                                                                     \
+        if (errp)                                                                                               \
+            lensed_render_wide_item<K, true>(d, cand, px, py, on, restage, blocks, quad, tables, npre, tab_lds, \
+                                             rays, model, errp);                                                \
+        else                                                                                                    \
+            lensed_render_wide_item<K, false>(d, cand, px, py, on, restage, blocks, quad, tables, npre,         \
+                                              tab_lds, rays, model, errp);                                      \
+        break;
+            LENSED_FOR_MODELS(LENSED_WIDE_CASE)
+#undef LENSED_WIDE_CASE
             default: break;
         }
     }
