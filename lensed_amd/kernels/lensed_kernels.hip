@@ -703,6 +703,7 @@ __device__ __attribute__((always_inline)) inline void lensed_epl_tables_block(
     float4* __restrict__ tables, const int* __restrict__ only)
 {
     __shared__ double nx[LENSED_EPL_ROWS], ny[LENSED_EPL_ROWS], ndx[LENSED_EPL_ROWS], ndy[LENSED_EPL_ROWS];
+    __shared__ double ratio[10];  // the series' coefficient ratios: ten divisions for the block, not for each node
     const int row0 = b * LENSED_EPL_ROWS;
     if (row0 >= nitems) return;
     int s = lensed_find_sys<4>(sys, nsys, row0);
@@ -712,10 +713,11 @@ __device__ __attribute__((always_inline)) inline void lensed_epl_tables_block(
     const float* p = params + d.param_off + (long long)cand * d.npar;
     const double q = p[d.epl_q], t = p[d.epl_t];
     const int i = (int)threadIdx.x;
-    lensed_epl_node(q, t, (double)i / LENSED_EPL_NT, nx[i], ny[i], ndx[i], ndy[i]);
+    if (i < 10) ratio[i] = lensed_epl_ratio(q, t, i + 1);
+    __syncthreads();
+    lensed_epl_node(ratio, t, (double)i / LENSED_EPL_NT, nx[i], ny[i], ndx[i], ndy[i]);
     if (i == 0)
-        lensed_epl_node(q, t, (double)LENSED_EPL_NT / LENSED_EPL_NT, nx[LENSED_EPL_NT], ny[LENSED_EPL_NT],
-                        ndx[LENSED_EPL_NT], ndy[LENSED_EPL_NT]);
+        lensed_epl_end(ratio, t, nx[LENSED_EPL_NT], ny[LENSED_EPL_NT], ndx[LENSED_EPL_NT], ndy[LENSED_EPL_NT]);
     __syncthreads();
     float4* out = tables + d.table_off + (long long)cand * LENSED_EPL_TABLE_F4;
     out[LENSED_EPL_AT(0, i)] = lensed_hermite(nx[i], ndx[i], nx[i + 1], ndx[i + 1]);
