@@ -61,28 +61,35 @@ __device__ inline void lensed_xcd_run(int n, int& first, int& end) {
 // parameters, written as a data block of LENSED_DWORDS words; with an EPL
 // table, also the lens-frame pair (F q_n, S q_n) of every quadrature node
 // offset, which the render kernel adds to the pixel's own part.
+// (nodes first, first + step, ...: one thread takes all, or a block's threads
+// share them)
 template <int K>
 __device__ inline void lensed_node_pairs(const lensed_desc& d, u32* blk, const float4* __restrict__ quad,
-                                         float4* __restrict__ npre, int cand)
+                                         float4* __restrict__ npre, int cand, int first, int step)
 {
     const float4* q = quad + d.quad_off;
-    const int pairs = d.table_mode ? d.nq : 0;
-    float4* out = npre + d.npre_off + (long long)cand * LENSED_NPRE_STRIDE(pairs);
-    for (int n = 0; n < pairs; ++n) {
+    float4* out = npre + d.npre_off + (long long)cand * LENSED_NPRE_STRIDE(d.nq);
+    for (int n = first; n < d.nq; n += step) {
         lcl::float4 v = lcl::epl_pre_model<K>(blk, lcl::float2(q[n].x, q[n].y), false);
         out[n] = make_float4(v.x, v.y, v.z, v.w);
     }
-    if (d.cull) {  // the candidate's constants of the pixel cull
-        lcl::float4 cc[LENSED_NPRE_CULL];
-        lcl::cull_consts_model<K>(blk, cc);
-        for (int i = 0; i < LENSED_NPRE_CULL; ++i) out[pairs + i] = make_float4(cc[i].x, cc[i].y, cc[i].z, cc[i].w);
-    }
+}
+
+// the candidate's constants of the pixel cull
+template <int K>
+__device__ inline void lensed_set_cull(const lensed_desc& d, u32* blk, float4* __restrict__ npre, int cand)
+{
+    const int pairs = d.table_mode ? d.nq : 0;
+    float4* out = npre + d.npre_off + (long long)cand * LENSED_NPRE_STRIDE(pairs) + pairs;
+    lcl::float4 cc[LENSED_NPRE_CULL];
+    lcl::cull_consts_model<K>(blk, cc);
+    for (int i = 0; i < LENSED_NPRE_CULL; ++i) out[i] = make_float4(cc[i].x, cc[i].y, cc[i].z, cc[i].w);
 }
 
 __device__ __attribute__((always_inline)) inline void lensed_set_params_item(
     const lensed_desc* __restrict__ sys, int nsys, int nitems, int item, const float* __restrict__ params,
     u32* __restrict__ blocks, const float4* __restrict__ quad, float4* __restrict__ npre, int* __restrict__ live,
-    int* __restrict__ owner, int layout)
+    int* __restrict__ owner, int layout, bool pairs)
 {
     if (item >= nitems) return;
     if (item == 0) {
@@ -104,8 +111,9 @@ __device__ __attribute__((always_inline)) inline void lensed_set_params_item(
 #define LENSED_SET_CASE(K)                                                \
     case K:                                                               \
         lcl::set_params_##K(blk, p);                                      \
-        if (d.table_mode || d.cull)                                       \
-            lensed_node_pairs<K>(d, blk, quad, npre, cand);               \
+        if (d.table_mode && pairs)                                        \
+            lensed_node_pairs<K>(d, blk, quad, npre, cand, 0, 1);         \
+        if (d.cull) lensed_set_cull<K>(d, blk, npre, cand);               \
         break;
         LENSED_FOR_MODELS(LENSED_SET_CASE)
 #undef LENSED_SET_CASE
@@ -123,7 +131,7 @@ extern "C" __global__ __launch_bounds__(256) void lensed_set_params(
     float4* __restrict__ npre, int* __restrict__ live, int* __restrict__ owner, int layout)
 {
     lensed_set_params_item(sys, nsys, nitems, (int)(blockIdx.x * blockDim.x + threadIdx.x), params, blocks, quad, npre,
-                           live, owner, layout);
+                           live, owner, layout, true);
 }
 
 // ------------------------------------------------------------------ render
@@ -698,9 +706,11 @@ extern "C" __global__ __launch_bounds__(LENSED_RENDER_BS) void lensed_cull(
 // systems' rows follow each other).  With `only` set, just the flagged
 // candidates (the emulator's fallback).
 static_assert(LENSED_EPL_NT == 256, "a table block has a thread per interval");
+template <bool PAIRS>
 __device__ __attribute__((always_inline)) inline void lensed_epl_tables_block(
     const lensed_desc* __restrict__ sys, int nsys, int nitems, int b, const float* __restrict__ params,
-    float4* __restrict__ tables, const int* __restrict__ only)
+    float4* __restrict__ tables, const int* __restrict__ only, const float4* __restrict__ quad,
+    float4* __restrict__ npre)
 {
     __shared__ double nx[LENSED_EPL_ROWS], ny[LENSED_EPL_ROWS], ndx[LENSED_EPL_ROWS], ndy[LENSED_EPL_ROWS];
     __shared__ double ratio[10];  // the series' coefficient ratios: ten divisions for the block, not for each node
@@ -714,6 +724,24 @@ __device__ __attribute__((always_inline)) inline void lensed_epl_tables_block(
     const double q = p[d.epl_q], t = p[d.epl_t];
     const int i = (int)threadIdx.x;
     if (i < 10) ratio[i] = lensed_epl_ratio(q, t, i + 1);
+    if (PAIRS && i < d.nq) {
+        // the candidate's node pairs, a thread per node: each forms the
+        // object block for itself (one thread per candidate took the nodes in
+        // turn and was the whole kernel's time, 21 us at 256 candidates, 9 so)
+        u32 blk[LENSED_DWORDS];
+#pragma unroll
+        for (int k = 0; k < LENSED_DWORDS; ++k) blk[k] = 0u;
+        switch (d.model) {
+#define LENSED_PAIRS_CASE(K)                                                          \
+    case K:                                                                           \
+        lcl::set_params_##K(blk, p);                                                  \
+        lensed_node_pairs<K>(d, blk, quad, npre, cand, i, LENSED_EPL_NT);             \
+        break;
+            LENSED_FOR_MODELS(LENSED_PAIRS_CASE)
+#undef LENSED_PAIRS_CASE
+            default: break;
+        }
+    }
     __syncthreads();
     lensed_epl_node(ratio, t, (double)i / LENSED_EPL_NT, nx[i], ny[i], ndx[i], ndy[i]);
     if (i == 0)
@@ -732,15 +760,16 @@ extern "C" __global__ __launch_bounds__(LENSED_EPL_NT) void lensed_epl_tables(
     const lensed_desc* __restrict__ sys, int nsys, int nitems,
     const float* __restrict__ params, float4* __restrict__ tables, const int* __restrict__ only)
 {
-    lensed_epl_tables_block(sys, nsys, nitems, (int)blockIdx.x, params, tables, only);
+    lensed_epl_tables_block<false>(sys, nsys, nitems, (int)blockIdx.x, params, tables, only, nullptr, nullptr);
 }
 
 // lensed_set_params and lensed_epl_tables (every candidate) in one launch:
 // the two read the parameters and write different buffers, so the first
 // set_blocks blocks are set_params' blocks and the rest the tables' blocks,
 // run side by side (set_params' one thread per candidate is latency-bound,
-// the tables' block per candidate fills the device meanwhile).  The same
-// code per thread as the two launches, so the same bits.
+// the tables' block per candidate fills the device meanwhile).  The tables'
+// blocks also form the node pairs, a thread per node, as lensed_set_params
+// does alone with a thread per candidate.
 extern "C" __global__ __launch_bounds__(LENSED_EPL_NT) void lensed_set_params_tables(
     const lensed_desc* __restrict__ sys, int nsys, int nitems,
     const float* __restrict__ params, u32* __restrict__ blocks, const float4* __restrict__ quad,
@@ -750,9 +779,9 @@ extern "C" __global__ __launch_bounds__(LENSED_EPL_NT) void lensed_set_params_ta
     const int b = (int)blockIdx.x;
     if (b < set_blocks)
         lensed_set_params_item(sys, nsys, nitems, b * LENSED_EPL_NT + (int)threadIdx.x, params, blocks, quad, npre,
-                               live, owner, layout);
+                               live, owner, layout, false);
     else
-        lensed_epl_tables_block(sys, nsys, ntable, b - set_blocks, params, tables, nullptr);
+        lensed_epl_tables_block<true>(sys, nsys, ntable, b - set_blocks, params, tables, nullptr, quad, npre);
 }
 
 // --------------------------------------------------------------- conv+chi2
