@@ -267,6 +267,9 @@ static int setup_params(System& S, const object* objs, size_t nobjs) {
 
 static hipFunction_t conv_function(const ::lensed* l, int rows);
 
+// parameters up to this size are read from pinned host memory (enqueue_chain)
+constexpr size_t kDirectParamBytes = 4096;
+
 static void free_layout(::lensed* l, Layout& L) {
     if (l->last_layout == &L) l->last_layout = nullptr;
     if (l->last_table_layout == &L) l->last_table_layout = nullptr;
@@ -570,7 +573,6 @@ static Buffers context_buffers(::lensed* l, const Layout& L) {
     B.blocks = l->d_blocks;
     B.model = l->d_model;
     B.partials = l->d_partials;
-    B.logl = l->d_logl;
     B.tables = l->d_tables;
     B.npre = l->d_npre;
     B.trace = l->d_trace;
@@ -599,11 +601,8 @@ static int enqueue_chain(::lensed* l, Layout& L, const Buffers& B, bool prof, fl
                          float* chi2_plane) {
     hipStream_t st = l->stream;
     auto rec = [&](int i) { if (prof) hipEventRecord(l->ev[i], st); };
-    size_t nparams = 0, nout = 0;
-    for (const auto& d : L.desc) {
-        nparams += (size_t)d.ncand * d.npar;
-        nout += d.ncand;
-    }
+    size_t nparams = 0;
+    for (const auto& d : L.desc) nparams += (size_t)d.ncand * d.npar;
     int nsys = (int)L.desc.size();
     // with a cull pass, the render walks the list of items it kept
     int* live = L.any_cull ? B.live : nullptr;
@@ -611,15 +610,24 @@ static int enqueue_chain(::lensed* l, Layout& L, const Buffers& B, bool prof, fl
     float* params = B.params;
     unsigned* blocks = B.blocks;
     float* model = B.model;
-    double* partials = B.partials;
-    double* logl = B.logl;
+    // the results go straight to pinned host memory: each candidate's logL,
+    // or, for a single candidate, its chi^2 partials, which the host adds up
+    // (finish_single) in less time than one more kernel takes to start
+    const bool single = L.n_final == 1;
+    double* partials = single ? l->h_partials : B.partials;
+    double* logl = l->h_logl;
     void* tables = B.tables;
     void* npre = B.npre;
     int* owner = B.owner;
     int* written = B.written;
     if (B.record) l->last_layout = &L;
     rec(0);
-    LSD_HIP(hipMemcpyAsync(params, l->h_params, nparams * sizeof(float), hipMemcpyHostToDevice, st));
+    // a few candidates' parameters are read by the kernels from the pinned
+    // buffer itself: a copy and the wait for it take longer (3 us a call)
+    if (nparams * sizeof(float) <= kDirectParamBytes)
+        params = l->h_params;
+    else
+        LSD_HIP(hipMemcpyAsync(params, l->h_params, nparams * sizeof(float), hipMemcpyHostToDevice, st));
     rec(1);
     rec(2);
     // with the emulator's network certified for some (q, t) cells, it builds
@@ -677,15 +685,26 @@ static int enqueue_chain(::lensed* l, Layout& L, const Buffers& B, bool prof, fl
         if (launch(f, grid, LENSED_CONV_BS, sweep ? 0 : L.lds_conv, st, a)) return -1;
     }
     rec(5);
-    {
+    if (!single) {
         void* a[] = {&desc, &nsys, &L.n_final, &partials, &logl};
         if (launch(l->f_final, (L.n_final + 3) / 4, 256, 0, st, a)) return -1;
     }
     rec(6);
-    LSD_HIP(hipMemcpyAsync(l->h_logl, logl, nout * sizeof(double), hipMemcpyDeviceToHost, st));
     rec(7);
     rec(8);
     return 0;
+}
+
+// lensed_finalize for the one candidate of a launch, on the host: the same
+// additions in the same order, a lane's partials 64 apart, then the lanes in
+// pairs 32, 16, ... apart
+static void finish_single(::lensed* l, const Layout& L) {
+    if (L.n_final != 1) return;
+    double lane[64] = {};
+    for (int t = 0; t < L.desc[0].npart; ++t) lane[t % 64] += l->h_partials[t];
+    for (int o = 32; o > 0; o >>= 1)
+        for (int i = 0; i < o; ++i) lane[i] += lane[i + o];
+    l->h_logl[0] = -0.5 * lane[0];
 }
 
 static int run_layout(::lensed* l, Layout& L) {
@@ -709,6 +728,7 @@ static int run_layout(::lensed* l, Layout& L) {
         return -1;
     }
     LSD_HIP(hipStreamSynchronize(l->stream));
+    finish_single(l, L);
     if (prof) {
         for (int i = 0; i < 8; ++i) {
             float ms = 0;
@@ -1124,11 +1144,13 @@ lensed* lensed_create(const lensed_system* systems, size_t nsys, const lensed_op
         l->cap_trace += l->max_batch * S.ntile_r * (LENSED_RENDER_BS / 64);
         l->cap_cull += l->max_batch * ((S.ntile_r + LENSED_CULL_GROUP - 1) / LENSED_CULL_GROUP);
     }
-    size_t maxpix = 0, dark_parts = 0;
+    size_t maxpix = 0, dark_parts = 0, max_parts = 1;
     for (auto& S : l->sys) {
         maxpix = std::max(maxpix, S.npix);
         S.dark_off = (long long)dark_parts;
-        dark_parts += ((S.height + 7) / 8) * ((S.width + LENSED_CONV_TX - 1) / LENSED_CONV_TX);
+        const size_t parts = ((S.height + 7) / 8) * ((S.width + LENSED_CONV_TX - 1) / LENSED_CONV_TX);
+        dark_parts += parts;
+        max_parts = std::max(max_parts, parts);
     }
     if (hipMalloc(&l->d_image, image.size() * 4) != hipSuccess ||
         hipMalloc(&l->d_weight, weight.size() * 4) != hipSuccess ||
@@ -1141,7 +1163,6 @@ lensed* lensed_create(const lensed_system* systems, size_t nsys, const lensed_op
         hipMalloc(&l->d_chi2, maxpix * 4) != hipSuccess ||
         hipMalloc(&l->d_partials, l->cap_partials * 8) != hipSuccess ||
         hipMalloc(&l->d_dark, dark_parts * 8) != hipSuccess ||
-        hipMalloc(&l->d_logl, l->cap_out * 8) != hipSuccess ||
         hipMalloc(&l->d_tables, std::max<size_t>(1, l->cap_tables) * 16) != hipSuccess ||
         hipMalloc(&l->d_npre, std::max<size_t>(1, l->cap_npre) * 16) != hipSuccess ||
         hipMalloc(&l->d_trace, std::max<size_t>(1, l->cap_trace) * 4) != hipSuccess ||
@@ -1154,7 +1175,8 @@ lensed* lensed_create(const lensed_system* systems, size_t nsys, const lensed_op
         hipHostMalloc(&l->h_flags, std::max<size_t>(1, l->cap_tables / LENSED_EPL_TABLE_F4) * 4,
                       hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc(&l->h_params, std::max<size_t>(1, l->cap_params) * 4, hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc(&l->h_logl, l->cap_out * 8, hipHostMallocDefault) != hipSuccess)
+        hipHostMalloc(&l->h_logl, l->cap_out * 8, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(&l->h_partials, max_parts * 8, hipHostMallocDefault) != hipSuccess)
         return fail("out of device memory");
     // on the context's stream (which, being non-blocking, would not wait for
     // the null stream), complete before the host vectors go
@@ -1213,13 +1235,14 @@ void lensed_destroy(lensed* l) {
     if (l->stream) hipStreamSynchronize(l->stream);
     for (auto& kv : l->layouts) free_layout(l, kv.second);
     void* bufs[] = {l->d_image, l->d_weight, l->d_psf, l->d_quad, l->d_params, l->d_blocks, l->d_model,
-                    l->d_err, l->d_conv, l->d_chi2, l->d_partials, l->d_logl, l->d_tables, l->d_nodes, l->d_npre,
+                    l->d_err, l->d_conv, l->d_chi2, l->d_partials, l->d_tables, l->d_nodes, l->d_npre,
                     l->d_flags, l->d_cells, l->emu_wf, l->emu_wp, l->d_trace, l->d_live, l->d_owner, l->d_written,
                     l->d_dark};
     for (void* b : bufs)
         if (b) hipFree(b);
     if (l->h_params) hipHostFree(l->h_params);
     if (l->h_logl) hipHostFree(l->h_logl);
+    if (l->h_partials) hipHostFree(l->h_partials);
     if (l->h_desc) hipHostFree(l->h_desc);
     if (l->h_flags) hipHostFree(l->h_flags);
     for (auto& e : l->ev)
@@ -1564,13 +1587,12 @@ int lensed_loglike_batch_noalloc(lensed* l, size_t s, const double* cubes, size_
                             d.table_mode ? nc * LENSED_EPL_TABLE_F4 * 16 : 16,
                             nc * (size_t)d.npix * 4,
                             nc * (size_t)d.npart * 8,
-                            nc * 8,
                             squares * 4,
                             live_capacity(squares, nc * ((d.ntile_r + LENSED_CULL_GROUP - 1) / LENSED_CULL_GROUP)) * 4,
                             squares * 4,
                             8};
-    size_t offs[12], total = 0;
-    for (int i = 0; i < 12; ++i) {
+    size_t offs[11], total = 0;
+    for (int i = 0; i < 11; ++i) {
         offs[i] = total;
         total += (sizes[i] + 255) / 256 * 256;
     }
@@ -1593,11 +1615,10 @@ int lensed_loglike_batch_noalloc(lensed* l, size_t s, const double* cubes, size_
     B.tables = base + offs[4];
     B.model = (float*)(base + offs[5]);
     B.partials = (double*)(base + offs[6]);
-    B.logl = (double*)(base + offs[7]);
-    B.trace = (int*)(base + offs[8]);
-    B.live = (int*)(base + offs[9]);
-    B.written = (int*)(base + offs[10]);
-    B.owner = (int*)(base + offs[11]);
+    B.trace = (int*)(base + offs[7]);
+    B.live = (int*)(base + offs[8]);
+    B.written = (int*)(base + offs[9]);
+    B.owner = (int*)(base + offs[10]);
     B.emulate = false;  // exact-series tables
     B.record = false;   // the context's own statistics are left alone
     // patch the layout to this call's count
@@ -1637,6 +1658,7 @@ int lensed_loglike_batch_noalloc(lensed* l, size_t s, const double* cubes, size_
     LSD_HIP(hipMemsetAsync(B.owner, 0xFF, 8, st));
     if (enqueue_chain(l, L, B, false, nullptr, nullptr, nullptr)) return -1;
     LSD_HIP(hipStreamSynchronize(st));
+    finish_single(l, L);
     for (size_t c = 0; c < nc; ++c)
         if (lnew_out[c] == 0.0) lnew_out[c] = l->h_logl[c];
     return 0;

@@ -103,7 +103,6 @@ struct Buffers {
     unsigned* blocks = nullptr;
     float* model = nullptr;
     double* partials = nullptr;
-    double* logl = nullptr;
     void* tables = nullptr;
     void* npre = nullptr;
     int* trace = nullptr;
@@ -145,7 +144,6 @@ struct lensed {
     float* d_conv = nullptr;    // convolved image, one candidate (dumper)
     float* d_chi2 = nullptr;    // per-pixel chi^2, one candidate (dumper)
     double* d_partials = nullptr;
-    double* d_logl = nullptr;
     void* d_tables = nullptr;   // EPL angular tables, float4 [candidates][LENSED_EPL_TABLE_F4]
     // EPL emulator: weights (fp32 and packed bf16), table nodes, per-candidate
     // choice (1 = exact series), the certified (q, t) cells, and the choice
@@ -166,6 +164,7 @@ struct lensed {
     // pinned host staging
     float* h_params = nullptr;
     double* h_logl = nullptr;
+    double* h_partials = nullptr;  // chi^2 partials of a single-candidate launch
     size_t block_pad = 4;  // words past the object blocks: every load takes a whole LENSED_DWORDS block
     size_t cap_params = 0, cap_blocks = 0, cap_model = 0, cap_partials = 0, cap_out = 0, cap_tables = 0;
     std::map<std::vector<size_t>, lsd::Layout> layouts;
