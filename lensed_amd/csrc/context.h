@@ -166,6 +166,8 @@ struct lensed {
     double* h_logl = nullptr;
     double* h_partials = nullptr;  // chi^2 partials of a single-candidate launch
     size_t block_pad = 4;  // words past the object blocks: every load takes a whole LENSED_DWORDS block
+    float* h_planes = nullptr;    // lensed_render's planes on their way to the caller (allocated by its first call)
+    hipEvent_t ev_plane[4] = {};
     size_t cap_params = 0, cap_blocks = 0, cap_model = 0, cap_partials = 0, cap_out = 0, cap_tables = 0;
     std::map<std::vector<size_t>, lsd::Layout> layouts;
     std::string source;          // generated program (for dumps)

@@ -244,7 +244,7 @@ class Context:
         """Dumper planes for one physical parameter vector (object order)."""
         spec = self.systems[s]
         h, w = spec.image.shape
-        planes = {k: np.zeros((h, w), dtype=np.float32) for k in ("value", "error", "image", "chi2")}
+        planes = {k: np.empty((h, w), dtype=np.float32) for k in ("value", "error", "image", "chi2")}  # filled by the call
         p = np.ascontiguousarray(phys, dtype=np.float64)
         fp = POINTER(c_float)
         _check(L.load().lensed_render(self.ptr, s, p.ctypes.data_as(POINTER(c_double)),
