@@ -49,7 +49,7 @@ inline float lensed_fract(float s) {
 inline float2 lensed_epl_w_tab(float2 u, float s, const float4* tab) {
     // p NT in [0, NT]; at u = 0 it is 0 * inf = NaN, which fmin turns into
     // NT (the end row: any finite W, since the power factor s^(1-t) decides)
-    float x = fminf(fabs(u.y) * ((float)LENSED_EPL_NT / s), (float)LENSED_EPL_NT);
+    float x = fminf(fabs(u.y) * ((float)LENSED_EPL_NT * recip(s)), (float)LENSED_EPL_NT);
     int i = (int)x;
     float f = lensed_fract(x);
     const float4 cx = tab[LENSED_EPL_AT(0, i)];

@@ -26,9 +26,9 @@ data
 static float2 deflection(local data* this, float2 x)
 {
     float2 u = mv22(this->fwd, x - this->c);
-    float w = sqrt(this->qq*u.x*u.x + u.y*u.y);
-    float ax = atan(this->ecc*u.x/(this->core + w));
-    float ay = atanh(this->ecc*u.y/(this->core*this->qq + w));
+    float w = lensed_sqrt(this->qq*u.x*u.x + u.y*u.y);
+    float ax = atan(this->ecc*u.x*recip(this->core + w));
+    float ay = atanh(this->ecc*u.y*recip(this->core*this->qq + w));
     return mv22(this->bwd, this->amp*(float2)(ax, ay));
 }
 

@@ -25,7 +25,7 @@ data
 static float2 deflection(local data* this, float2 x)
 {
     float2 u = mv22(this->fwd, x - this->c);
-    float s = this->ecc/sqrt(this->qq*u.x*u.x + u.y*u.y);
+    float s = this->ecc*rsqrt(this->qq*u.x*u.x + u.y*u.y);
     return mv22(this->bwd, this->amp*(float2)(atan(u.x*s), atanh(u.y*s)));
 }
 

@@ -27,7 +27,7 @@ static float2 deflection(local data* this, float2 x)
 {
     float2 d = x - this->c;
     float2 u = mv22(this->fwd, d);
-    float s = this->ecc/sqrt(this->qq*u.x*u.x + u.y*u.y);
+    float s = this->ecc*rsqrt(this->qq*u.x*u.x + u.y*u.y);
     return mv22(this->bwd, this->amp*(float2)(atan(u.x*s), atanh(u.y*s))) + mv22(this->shear, d);
 }
 
