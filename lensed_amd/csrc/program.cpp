@@ -348,12 +348,9 @@ static bool slope_culls(const std::vector<ModelObject>& objs) {
 }
 
 bool model_holds(const std::vector<ModelObject>& objs) {
-    // at most 64 words, so that the loop stays within its 128 registers; not
-    // with an EPL series per ray (lensed_render_item has both sides measured)
-    if (model_data_words(objs) > 64) return false;
-    for (const auto& ob : objs)
-        if (ob.type == OBJ_LENS && !ob.table && object_tabulates(ob.name)) return false;
-    return true;
+    // at most 64 words, so that the loop stays within its 128 registers: 16
+    // systems of larger models take 16.1 ms held and 15.9 as scalars
+    return model_data_words(objs) <= 64;
 }
 
 bool model_culls(const std::vector<ModelObject>& objs) { return frame_culls(objs) || slope_culls(objs); }

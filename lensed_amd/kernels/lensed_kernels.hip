@@ -162,14 +162,14 @@ __device__ inline bool lensed_list_pixel(const lensed_desc& d, int cand, int q, 
 // One thread per pixel (px, py; on: the thread has one); the 2-D quadrature
 // loop runs in the thread with the node table in scalar registers.  The
 // candidate's object block is wave-uniform and comes in by scalar loads; for
-// most models it is then held in vector registers (model_holds): multiplies,
-// adds and FMAs of vector registers and literals issue at up to 1.75 per CU
-// and cycle, those with a scalar operand at 0.93.  Measured over the ray
-// loops, cycles of a CU per wave and ray, scalar and vector: SIE + Sersic 202
-// and 182, SIE + shear + two sources + sky 203 and 183, tabulated EPL + two
-// Sersic + sky 73.7 and 70.2, tabulated EPL + Gaussian 41.5 and 39.2.  The EPL
-// series, which takes a coefficient per Horner step and is half fast
-// instructions either way, loses: 81.5 and 84 (not held).
+// models of up to 64 words it is then held in vector registers (model_holds):
+// multiplies, adds and FMAs of vector registers and literals issue at up to
+// 1.75 per CU and cycle, those with a scalar operand at 0.93.  Measured,
+// scalar and vector, the whole stage: tabulated EPL + two Sersic + sky, 512
+// candidates of 512x512, 9.87 and 8.46 ms; an EPL's series + Sersic, 512 of
+// 256x256, 0.592 and 0.552 ms; cored SIE + two Sersic, 256 of 131x97, 0.873
+// and 0.848 ms; tabulated EPL + Sersic, 4096 of 256x256, 1.98 and 1.96 ms; SIE
+// + Sersic, 256 of 100x100, and SIE + shear, 1024 of 200x200, within 1 %.
 // (The block is read whole, LENSED_DWORDS words, in a few wide scalar loads;
 // the words past a smaller model's own are not used, and the host keeps that
 // much room after the last block.)
