@@ -340,7 +340,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
     // waves per SIMD each strip is cut into parts, a wave each, at the price
     // of refilling the window above every part (256 candidates whole, in 2, 4
     // and 8 parts: 70, 45, 41 and 50 us; 1024: 93, 92, 112 and 126).
-    bool sweep_ok = true, all_culled = true;
+    bool sweep_ok = true, all_culled = true, some_culled = false;
     long long strips = 0;
     for (size_t s = 0; s < l->sys.size(); ++s) {
         const System& S = l->sys[s];
@@ -349,7 +349,10 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         if (!S.psfw || S.sep_rank != 1 || S.psfw > LENSED_SWEEP_MAX_PSF || S.psfh > LENSED_SWEEP_MAX_PSF ||
             S.height > LENSED_SWEEP_MAX_H)
             sweep_ok = false;
-        if (!S.cull || no_cull) all_culled = false;
+        if (!S.cull || no_cull)
+            all_culled = false;
+        else
+            some_culled = true;
     }
     if (!tq.conv_rows && sweep_ok && all_culled && strips >= 2LL * l->cu_count) L.conv_rows = LENSED_CONV_SWEEP;
     if (L.conv_rows == LENSED_CONV_SWEEP && !sweep_ok)
@@ -389,7 +392,14 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         d.psfh = (int)S.psfh;
         d.ncand = (int)ncand[s];
         d.npar = (int)S.pars.size();
-        d.ntile_r = S.ntile_r;
+        // no block is cut off by the image's edge if items are pixels in a
+        // row; the cull's list and flags, where the launch has them, are of
+        // 16 x 16 blocks.  (us, blocks and rows: 256 candidates of 100 x 100
+        // 500, 442; 256 of 131 x 97 847, 795; 1024 of 200 x 200 7325, 7120;
+        // 139 of 186 x 154 695, 639; tabulated, 1803 of 123 x 170 1963, 1873)
+        const int in_rows = (int)((S.npix + LENSED_RENDER_BS - 1) / LENSED_RENDER_BS);
+        d.linear = !some_culled && in_rows < S.ntile_r ? 1 : 0;
+        d.ntile_r = d.linear ? in_rows : S.ntile_r;
         d.dwords = (int)S.dwords;
         d.conv_ry = ry;
         d.tiles_x = (int)((S.width + LENSED_CONV_TX - 1) / LENSED_CONV_TX);
@@ -433,6 +443,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         partial_off += nc * d.npart;
         out_off += nc;
         ir += (int)(nc * d.ntile_r);
+        L.n_blocks += (long)(nc * S.ntile_r);
         ik += (int)(nc * ((d.ntile_r + LENSED_CULL_GROUP - 1) / LENSED_CULL_GROUP));
         ic += (int)(nc * (sweep ? d.tiles_x * seg : d.ntile_c));  // sweep: an item per part of a 64-column strip
         is += (int)nc;
@@ -1392,7 +1403,7 @@ int lensed_render_stats(const lensed* l, long* items, long* listed, long* quads,
         return -1;
     }
     const Layout& L = *l->last_layout;
-    const long n = L.n_render, per = LENSED_RENDER_BS / 64;
+    const long n = L.n_blocks, per = LENSED_RENDER_BS / 64;  // (without a cull the items may be pixels in a row)
     long nl = n, nq = 16 * n;
     if (L.any_cull && (listed || quads)) {
         // the cull's list: quads (item * 4 + w) * 4 + q, sixteen to an entry,

@@ -75,6 +75,7 @@ struct Layout {
     std::vector<lensed_desc> desc;  // systems with ncand > 0
     std::vector<int> sys_of_desc;
     int n_set = 0, n_render = 0, n_cull = 0, n_conv = 0, n_final = 0, n_table = 0;
+    long n_blocks = 0;  // 16 x 16 blocks of the launch's images: n_render but for linear systems
     int n_nodes = 0, n_tcands = 0;  // emulator: table nodes and candidates with a table
     size_t lds_conv = 0, lds_render = 0;
     bool conv_small = false;        // short tiles: launch too small to fill the GPU

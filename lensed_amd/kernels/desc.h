@@ -58,7 +58,8 @@ struct lensed_desc {
     long long npre_off;                  // float4 into npre[]: node pairs, cull constants ([ncand][pairs + 3])
     float qrad;                          // largest distance of a quadrature node from the pixel centre
     int cull;                            // skip pixels whose rays provably all miss the source
-    int sweep_seg, pad_;                 // column sweep: waves per 64-column strip, each a part of its rows
+    int sweep_seg, linear;               // column sweep: waves per 64-column strip, each a part of its rows;
+                                         // render items of 256 pixels in a row, not 16 x 16 blocks
     long long dark_off;                  // doubles into the data's chi^2 block partials for a model of 0 ([npart])
 };
 
