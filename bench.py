@@ -31,11 +31,12 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 METRIC = "logL evals/sec at 256² px, batched+emulated vs plain GPU, |ΔlogL|≤0.01"
-PEAK_FP32_NONPACKED = 78.6  # TFLOP/s: one wave64 FMA per CU per cycle (packed FP32 is not used)
+PEAK_FP32_NONPACKED = 78.6  # TFLOP/s: one wave64 FMA per CU per cycle, nominal (packed FP32 is not used)
 PEAK_HBM = 8000.0  # GB/s
-# The render kernel is bound by VALU issue: one wave64 VALU instruction per
-# CU per cycle, 256 CUs at 2.4 GHz
-VALU_ISSUE_PEAK = 256 * 2.4e9  # wave instructions per second
+# The render kernel is bound by VALU issue: at best 1.75 wave64 VALU
+# instructions per CU per cycle (measured: multiplies, adds and FMAs of vector
+# registers and literals; 0.93 with a scalar operand), 256 CUs at 2.4 GHz
+VALU_ISSUE_PEAK = 1.75 * 256 * 2.4e9  # wave instructions per second
 # reference-formula work of this workload (add/mul/div 1, FMA 2,
 # transcendental 1): 165 flop per ray, 49 rays per pixel
 REF_FLOP_PER_RAY = 165
@@ -212,18 +213,18 @@ def render_roofline(kt, tr, K):
                 "note": "FP32 flop the kernel executes, from the rocprofv3 SQ_INSTS_VALU_FMA_F32 (x2), ADD_F32, "
                         "MUL_F32 and TRANS_F32 counts of the seeded launch (x64 lanes) per traced quad, over "
                         "this run's quads and kernel time; the published 157.3 TFLOP/s counts packed FP32, "
-                        "which the build disables, so one FP32 operation per lane per cycle (78.6 TFLOP/s) is "
-                        "the ceiling here and the ray's non-FP32 work (LDS, conversions, copysigns) issues "
-                        "between them"},
+                        "which the build disables; 78.6 TFLOP/s is one FP32 operation per lane per cycle, nominal "
+                        "(multiplies, adds and FMAs of vector registers alone reach 1.75), and the ray's "
+                        "non-FP32 work (LDS, conversions, copysigns) issues between them"},
             "reference_flop_equivalent": {
                 "tflops": round(REF_FLOP_PER_RAY * rays / s / 1e12, 2),
                 "note": "the reference formulas' 165 flop per traced ray (its tenth-order series); the table "
                         "path computes the same ray in fewer instructions, so this rate is not a fraction of "
                         "any hardware peak"},
-            "note": "frac = non-transcendental VALU wave instructions issued / (256 CUs x 2.4 GHz x kernel "
-                    "time), the nominal issue peak of the VALU (one wave64 instruction per CU per cycle); at "
-                    "the clock the kernel runs (GRBM_GUI_ACTIVE in the profile) it issues 0.95 of them per CU "
-                    "per cycle, with the transcendentals on their own unit beside them"}
+            "note": "frac = non-transcendental VALU wave instructions issued / (1.75 x 256 CUs x 2.4 GHz x "
+                    "kernel time): 1.75 per CU per cycle is the measured rate of multiplies, adds and FMAs "
+                    "of vector registers alone; comparisons, conversions and scalar operands issue at 0.93, "
+                    "and the transcendentals go beside them"}
 
 
 def conv_roofline(kt, K, conv_rows, npix=65536, taps=21):
@@ -627,7 +628,7 @@ def main():
                           "path": "batched, per-ray tenth-order EPL series"},
         "accuracy_vs_exact": acc,
         "plain_gpu": {"value": round(plain_rate, 2), "unit": "logL evals/s",
-                      "path": "one candidate per loglike() call, 4 kernels + 2 copies + sync",
+                      "path": "one candidate per loglike() call, 4 kernels + sync, parameters and logL through pinned memory",
                       "identical_logL_to_batched": same},
         "speedup_vs_plain": round(value / plain_rate, 3),
         "roofline": render_roofline(kt, tr, K),

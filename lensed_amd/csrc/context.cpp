@@ -395,7 +395,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         // no block is cut off by the image's edge if items are pixels in a
         // row; the cull's list and flags, where the launch has them, are of
         // 16 x 16 blocks.  (us, blocks and rows: 256 candidates of 100 x 100
-        // 500, 442; 256 of 131 x 97 847, 795; 1024 of 200 x 200 7325, 7120;
+        // 500, 442; 333 of 131 x 97 847, 795; 1024 of 200 x 200 7325, 7120;
         // 139 of 186 x 154 695, 639; tabulated, 1803 of 123 x 170 1963, 1873)
         const int in_rows = (int)((S.npix + LENSED_RENDER_BS - 1) / LENSED_RENDER_BS);
         d.linear = !some_culled && in_rows < S.ntile_r ? 1 : 0;

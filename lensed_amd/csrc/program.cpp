@@ -348,8 +348,8 @@ static bool slope_culls(const std::vector<ModelObject>& objs) {
 }
 
 bool model_holds(const std::vector<ModelObject>& objs) {
-    // at most 64 words, so that the loop stays within its 128 registers: 16
-    // systems of larger models take 16.1 ms held and 15.9 as scalars
+    // at most 64 words, so that the block and the ray's own values (about 50
+    // registers with two sources) stay within the loop's 128 registers
     return model_data_words(objs) <= 64;
 }
 

@@ -176,9 +176,9 @@ __device__ inline bool lensed_list_pixel(const lensed_desc& d, int cand, int q, 
 // multiplies, adds and FMAs of vector registers and literals issue at up to
 // 1.75 per CU and cycle, those with a scalar operand at 0.93.  Measured,
 // scalar and vector, the whole stage: tabulated EPL + two Sersic + sky, 512
-// candidates of 512x512, 9.87 and 8.46 ms; an EPL's series + Sersic, 512 of
-// 256x256, 0.592 and 0.552 ms; cored SIE + two Sersic, 256 of 131x97, 0.873
-// and 0.848 ms; tabulated EPL + Sersic, 4096 of 256x256, 1.98 and 1.96 ms; SIE
+// candidates of 512x512, 9.87 and 8.46 ms; an EPL's series + Gaussian, 512 of
+// 256x256, 0.592 and 0.552 ms; cored SIE + exponential, 333 of 131x97, 0.873
+// and 0.848 ms; tabulated EPL + Gaussian, 4096 of 256x256, 1.98 and 1.96 ms; SIE
 // + Sersic, 256 of 100x100, and SIE + shear, 1024 of 200x200, within 1 %.
 // (The block is read whole, LENSED_DWORDS words, in a few wide scalar loads;
 // the words past a smaller model's own are not used, and the host keeps that

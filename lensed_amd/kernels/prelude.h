@@ -145,10 +145,10 @@ LCL_F1(log1p, ::log1pf)
 // one inside ::atanhf cannot be reached.  The empty statements on the
 // results keep atan's code before atanh's: interleaved, they measure 12 % more.
 // The rendering stage without and with, in ms: 256 singular isothermal
-// ellipsoids at 100x100, 3x3 rays: 0.56 and 0.51 (the whole of atan and atanh
-// raised: 0.54); 256 cored ones at 131x97, two sources: 1.10 and 0.87 (1.01);
-// 1024 in shear at 200x200, 5x5 rays: 8.1 and 7.05 (7.46); 16 systems of such
-// lenses, 64 candidates each: 19.6 and 16.5 (18.3).  In cycles of a CU per 64
+// ellipsoids at 100x100, 49 rays: 0.56 and 0.51 (the whole of atan and atanh
+// raised: 0.54); 333 cored ones at 131x97: 1.10 and 0.87 (1.01); 1024 in shear
+// at 200x200, two sources: 8.1 and 7.05 (7.46); 16 systems of SIEs or EPL
+// series, 64 candidates each: 19.6 and 16.5 (18.3).  In cycles of a CU per 64
 // rays: an EPL's series 84 and 75, a table of it at 256x256 39.2 and 37.3, at
 // 512x512 70.2 and 61.1.
 #if defined(__HIP_DEVICE_COMPILE__)
