@@ -296,6 +296,18 @@ static void evict_layouts(::lensed* l) {
 // everything of a launch layout but its device descriptors (no allocation
 // on the device); 0 on success
 static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L) {
+    size_t total = 0;
+    for (size_t s = 0; s < l->sys.size(); ++s) {
+        if (ncand[s] > l->max_batch) {
+            set_error("more candidates than max_batch");
+            return -1;
+        }
+        total += ncand[s];
+    }
+    if (total == 0) {
+        set_error("no candidates");
+        return -1;
+    }
     // conv tile height: the tallest of which the launch has two per CU.  (us,
     // 8-, 32- and 64-row tiles, by the number of 64-row ones: direct 31 x 31
     // taps 256: 46, 41, 47; 512: 84, 66, 52; 32768: 4782, 3782, 2750; two
@@ -378,10 +390,6 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
     for (size_t s = 0; s < l->sys.size(); ++s) {
         if (!ncand[s]) continue;
         const System& S = l->sys[s];
-        if (ncand[s] > l->max_batch) {
-            set_error("more candidates than max_batch");
-            return -1;
-        }
         lensed_desc d;
         memset(&d, 0, sizeof d);
         d.width = (int)S.width;
@@ -464,10 +472,6 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         }
         L.desc.push_back(d);
         L.sys_of_desc.push_back((int)s);
-    }
-    if (L.desc.empty()) {
-        set_error("no candidates");
-        return -1;
     }
     // persistent grids sized by what stays resident with this launch's LDS,
     // times the requested multiples.  The render's default is 16 times over

@@ -1,0 +1,71 @@
+"""The host's launch code on the CPU: a child process with a HIP runtime
+without a device preloaded (hip_stub.cpp), whose kernels do nothing."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+from conftest import ROOT
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes, sys
+sys.path[:0] = [%r, %r]
+import numpy as np
+from lensed_amd import _lib as L
+from lensed_amd.lensed import Context, LensedError, SystemSpec
+stub = ctypes.CDLL(None)
+stub.stub_log.restype = ctypes.c_char_p
+
+def launches():
+    lines = [s.split() for s in stub.stub_log().decode().splitlines()]
+    stub.stub_clear()
+    return {name: (int(blocks), int(lds)) for name, blocks, lds in lines}
+
+def spec(lens, source, shape, psf=None):
+    params = {"sie": "x y r q pa", "epl_plus_shear": "x y r t q pa g1 g2", "gauss": "x y sigma mag q pa",
+              "sersic": "x y r mag n q pa"}
+    pri = {f"{o}.{p}": "unif 0.5 1" for o, n in (("lens", lens), ("source", source)) for p in params[n].split()}
+    return SystemSpec([("lens", lens), ("source", source)], pri, np.zeros(shape, np.float32),
+                      np.ones(shape, np.float32), psf=psf)
+""" % (ROOT, HERE)
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    d = tmp_path_factory.mktemp("stub")
+    so = str(d / "hip_stub.so")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__",
+                           "-I/opt/rocm/include", "-o", so,
+                           os.path.join(HERE, "hip_stub.cpp")])
+
+    def call(code):
+        env = dict(os.environ, LD_PRELOAD=so, LENSED_CACHE_DIR=str(d))
+        r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(code)], env=env, capture_output=True,
+                           text=True, timeout=300)
+        assert r.returncode == 0, (r.returncode, r.stderr[-3000:])
+        return r.stdout
+    return call
+
+
+@pytest.mark.parametrize("lens", ["sie", "epl_plus_shear"])
+def test_a_launch_without_candidates_is_an_error(run, lens):
+    run(f"""
+    with Context([spec({lens!r}, "gauss", (20, 30)), spec("sie", "sersic", (16, 16))], max_batch=4) as ctx:
+        for counts in ([0, 0], [5, 0], [0, 1 << 62]):
+            out = np.zeros(8)
+            DP = ctypes.POINTER(ctypes.c_double)
+            p = np.zeros(200)
+            rc = L.load().lensed_loglike_systems(ctypes.c_void_p(ctx.ptr), (DP * 2)(*[p.ctypes.data_as(DP)] * 2),
+                                                 (ctypes.c_size_t * 2)(*counts), (DP * 2)(*[out.ctypes.data_as(DP)] * 2))
+            assert rc != 0 and ("no candidates" if not any(counts) else "max_batch") in L.last_error(), L.last_error()
+        try:
+            ctx.loglike_phys([np.zeros((0, ctx.npars(0))), np.zeros((0, ctx.npars(1)))])
+            raise SystemExit("no error")
+        except LensedError as e:
+            assert "no candidates" in str(e)
+        assert ctx.loglike_phys([np.zeros((0, ctx.npars(0))), np.full((2, ctx.npars(1)), 0.7)])[1].shape == (2,)
+    """)
