@@ -37,7 +37,7 @@ static float deflection_slope(local data* this, float2 x, float rho)
     float2 d = x - this->c;
     float2 u = mv22(this->fwd, d);
     float w = sqrt(this->qq*u.x*u.x + u.y*u.y) - rho;
-    return w > 0 ? this->amp*this->ecc/w : HUGE_VALF;
+    return w > 0 ? fabs(this->amp*this->ecc)/w : HUGE_VALF;
 }
 
 static void set(local data* this, float x, float y, float r, float q, float pa)

@@ -93,6 +93,32 @@ def test_slope_cull_never_skips_a_lit_ray(lens, nsrc):
     assert skipped > 1000, skipped
 
 
+# what the parameters' bounds leave out but loglike_phys and render take: a
+# negative Einstein radius (a deflection outwards), a negative sigma
+@pytest.mark.parametrize("lens", list(LENS))
+@pytest.mark.parametrize("r,sigma", [(-10.0, 1.0), (-10.0, -1.0), (10.0, -1.0), (-4.0, 0.4), (-30.0, 3.0)])
+def test_slope_cull_with_negative_radii(lens, r, sigma):
+    lib = _host([("lens", lens), ("s", "gauss")])
+    qq, _ = Q.rule("g3k7")
+    qn = np.ascontiguousarray(np.asarray(qq, np.float32).reshape(-1, 2))
+    rho = float(np.hypot(qn[:, 0], qn[:, 1]).max() * (1 + 1e-6))
+    rng = np.random.default_rng(23)
+    fp = POINTER(c_float)
+    out = (c_int * 2)()
+    skipped = 0
+    for it in range(8):
+        v = {"x": rng.uniform(45, 56), "y": rng.uniform(45, 56), "r": r * rng.uniform(0.7, 1.3),
+             "t": rng.uniform(0.3, 1.7), "q": rng.uniform(0.2, 0.95), "pa": rng.uniform(0, 180),
+             "g1": rng.uniform(-0.2, 0.2), "g2": rng.uniform(-0.2, 0.2)}
+        s = {"x": rng.uniform(40, 60), "y": rng.uniform(40, 60), "sigma": sigma, "mag": rng.uniform(-8, 5),
+             "q": rng.uniform(0.3, 1), "pa": rng.uniform(0, 180)}
+        params = np.array([v[p] for p in LENS[lens]] + [s[p] for p in GAUSS], np.float32)
+        lib.host_cull(params.ctypes.data_as(fp), 100, 100, qn.ctypes.data_as(fp), len(qn), rho, out)
+        assert out[1] == 0, (it, params, list(out))
+        skipped += out[0]
+    assert skipped  # (a lens of -30 pixels with t < 1 spreads a wide source over most of the image)
+
+
 def test_models_that_take_the_slope_cull():
     """Lenses first, then compact sources alone; anything else (a sky, a
     source with a far cutoff, a source before the lens, a lens without a
