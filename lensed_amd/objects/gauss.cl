@@ -37,10 +37,12 @@ static float frame_profile(local data* this, float2 u)
 
 // |u| beyond which frame_profile is below 2^-127: a subnormal, which the
 // kernels' FP32 arithmetic (subnormals flushed, as the reference's
-// -cl-denorms-are-zero) takes as 0, so the ray adds exactly nothing
+// -cl-denorms-are-zero) takes as 0, so the ray adds exactly nothing (a NaN
+// stays one: that brightness is NaN everywhere, and no pixel lies beyond it)
 static float frame_cutoff(local data* this)
 {
-    return sqrt(fmax(this->lpk + 127, 0.0f));
+    float e = this->lpk + 127;
+    return e <= 0 ? 0.0f : sqrt(e);
 }
 
 // the cutoff is about 13 sigma out: most pixels of an image lie beyond it

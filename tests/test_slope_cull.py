@@ -119,6 +119,21 @@ def test_slope_cull_with_negative_radii(lens, r, sigma):
     assert skipped  # (a lens of -30 pixels with t < 1 spreads a wide source over most of the image)
 
 
+# a brightness that is no number is one at every ray: nothing may be skipped
+@pytest.mark.parametrize("lens", list(LENS))
+@pytest.mark.parametrize("bad", [{"mag": np.nan}, {"q": -0.5}, {"sigma": np.nan}, {"mag": -np.inf}])
+def test_slope_cull_keeps_what_is_not_a_number(lens, bad):
+    lib = _host([("lens", lens), ("s", "gauss")])
+    v = {"x": 50.0, "y": 51.0, "r": 10.0, "t": 1.1, "q": 0.7, "pa": 30.0, "g1": 0.05, "g2": -0.02}
+    s = {"x": 49.0, "y": 53.0, "sigma": 0.5, "mag": 0.0, "q": 0.6, "pa": 70.0, **bad}
+    params = np.array([v[p] for p in LENS[lens]] + [s[p] for p in GAUSS], np.float32)
+    qn = np.zeros((1, 2), np.float32)
+    fp = POINTER(c_float)
+    out = (c_int * 2)()
+    lib.host_cull(params.ctypes.data_as(fp), 100, 100, qn.ctypes.data_as(fp), 1, 0.8, out)
+    assert out[1] == 0, list(out)
+
+
 def test_models_that_take_the_slope_cull():
     """Lenses first, then compact sources alone; anything else (a sky, a
     source with a far cutoff, a source before the lens, a lens without a
