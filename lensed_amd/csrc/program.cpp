@@ -15,6 +15,7 @@
 #include <dlfcn.h>
 #include <sys/stat.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <fstream>
@@ -255,9 +256,24 @@ static std::string plugin_text(const std::string& name) {
     return src;
 }
 
+// comments as blanks: they may hold braces, and functions left out
+static std::string without_comments(const std::string& src) {
+    std::string out;
+    for (size_t i = 0; i < src.size();) {
+        const size_t c = std::min(src.find("/*", i), src.find("//", i));
+        out.append(src, i, c == std::string::npos ? c : c - i);
+        if (c == std::string::npos) break;
+        const bool block = src[c + 1] == '*';
+        const size_t e = src.find(block ? "*/" : "\n", c + 2);
+        out += ' ';
+        i = e == std::string::npos ? src.size() : block ? e + 2 : e;
+    }
+    return out;
+}
+
 // whether a plugin defines the functions named by the patterns
 static bool plugin_defines(const std::string& name, const std::vector<const char*>& patterns) {
-    const std::string src = plugin_text(name);
+    const std::string src = without_comments(plugin_text(name));
     bool ok = !src.empty();
     for (const char* re : patterns) ok = ok && std::regex_search(src, std::regex(re));
     return ok;
@@ -265,10 +281,7 @@ static bool plugin_defines(const std::string& name, const std::vector<const char
 
 // whether the plugin's data block declares every field of the patterns
 static bool data_declares(const std::string& name, const std::vector<const char*>& fields) {
-    // comments removed first: they may hold braces
-    const std::string src =
-        std::regex_replace(std::regex_replace(plugin_text(name), std::regex(R"(/\*[\s\S]*?\*/)"), " "),
-                           std::regex(R"(//[^\n]*)"), " ");
+    const std::string src = without_comments(plugin_text(name));
     std::smatch m;
     if (!std::regex_search(src, m, std::regex(R"(\bdata\s*\{([^}]*)\})"))) return false;
     const std::string block = m[1].str();
@@ -321,9 +334,10 @@ static bool frame_culls(const std::vector<ModelObject>& objs) {
 }
 
 // The image-frame cull: one plane of lenses, none tabulated, each with a
-// bound on its own slope, then sources that end within a few scale lengths
-// (frame_compact).  Sources with a cutoff tens of scale lengths out (Sersic,
-// exponential) light nearly every pixel: for them the pass would only cost.
+// bound on its own slope, then sources that may end within a few scale
+// lengths (frame_compact; one that returns false keeps every pixel).  Sources
+// with a cutoff tens of scale lengths out (Sersic, exponential) light nearly
+// every pixel: for them the pass would only cost.
 // The render traces at the VALU's issue rate, so skipped rays are saved in
 // full: 512 candidates of 256 x 256, EPL + shear by its series and a Gaussian
 // source, 3.48 ms a launch tracing every ray, 0.77 ms culled.
@@ -500,6 +514,14 @@ std::string compute_function(const std::vector<ModelObject>& objs, int k) {
     else if (slopes) {
         o << "    const float2 x = float2(base.x, base.y);\n    float2 a = 0;\n    float slope = 1.0f;\n";
         size_t at = 0, n = 0;
+        for (const auto& ob : objs) {
+            if (ob.type == OBJ_SOURCE) {
+                const std::string m = mangle(ob.name);
+                o << "    if (!frame_compact_" << m << "(" << data_ptr(m, at, "data") << ")) return false;\n";
+            }
+            at += ob.size;
+        }
+        at = 0;
         for (const auto& ob : objs) {
             const std::string m = mangle(ob.name), p = data_ptr(m, at, "data");
             if (ob.type == OBJ_LENS)

@@ -134,6 +134,28 @@ def test_slope_cull_keeps_what_is_not_a_number(lens, bad):
     assert out[1] == 0, list(out)
 
 
+def test_plugins_say_whether_they_are_culled(tmp_path, monkeypatch):
+    """frame_compact's value counts, and a function in a comment is none."""
+    objs = os.path.join(os.path.dirname(L.__file__), "objects")
+    gauss, sie = (open(os.path.join(objs, n + ".cl")).read() for n in ("gauss", "sie"))
+    head, body = gauss.split("static bool frame_compact", 1)
+    (tmp_path / "broad.cl").write_text(head + "static bool frame_compact" + body.replace("return true;", "return false;", 1))
+    head, body = sie.split("static float deflection_slope", 1)
+    old, rest = body.split("\n}\n", 1)
+    (tmp_path / "plain.cl").write_text(head + "/* static float deflection_slope" + old + "\n}\n*/" + rest)
+    monkeypatch.setenv("LENSED_OBJECTS_PATH", str(tmp_path))
+    qn = np.zeros((1, 2), np.float32)
+    params = np.array([50.0, 51.0, 10.0, 0.7, 30.0, 49.0, 53.0, 0.5, 0.0, 0.6, 70.0], np.float32)
+    fp = POINTER(c_float)
+    out = (c_int * 2)()
+    for source in ("gauss", "broad"):
+        _host([("lens", "sie"), ("s", source)]).host_cull(params.ctypes.data_as(fp), 100, 100, qn.ctypes.data_as(fp), 1,
+                                                          0.8, out)
+        assert (out[0] > 0) == (source == "gauss"), (source, list(out))
+    pair = [("lens", "plain"), ("s", "gauss")]
+    assert "lensed_slope_cull(" not in L.take_string(L.load().lensed_model_source(2, load_objects(pair))).split("cull_0", 1)[1]
+
+
 def test_models_that_take_the_slope_cull():
     """Lenses first, then compact sources alone; anything else (a sky, a
     source with a far cutoff, a source before the lens, a lens without a
