@@ -560,20 +560,6 @@ static Layout* get_layout(::lensed* l, const std::vector<size_t>& ncand, bool em
     return &(l->layouts[key] = L);
 }
 
-// one layout per system for lensed_loglike_batch_noalloc, built for
-// max_batch candidates and patched to a call's count (a single system's
-// offsets into its buffers are all zero)
-static int build_noalloc_layouts(::lensed* l) {
-    l->noalloc.assign(l->sys.size(), Layout());
-    for (size_t s = 0; s < l->sys.size(); ++s) {
-        std::vector<size_t> nc(l->sys.size(), 0);
-        nc[s] = l->max_batch;
-        if (build_layout(l, nc, l->noalloc[s])) return -1;
-        l->noalloc[s].id = -2;  // never the id a fill of `owner` leaves (-1)
-    }
-    return 0;
-}
-
 // ints of the cull's render list: the count, the quads (four per square),
 // and the pads (fewer than an entry per cull block, where a block's part of
 // a candidate ends; a launch has no more blocks than cull items)
@@ -1236,12 +1222,7 @@ lensed* lensed_create(const lensed_system* systems, size_t nsys, const lensed_op
             hipMemcpy(l->d_cells, cells.data(), cells.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
             return fail("emulator cells");
     }
-    if (build_noalloc_layouts(l)) {
-        std::string e = lsd::g_error;
-        lensed_destroy(l);
-        set_error(e);
-        return nullptr;
-    }
+    l->noalloc.assign(l->sys.size(), Layout());
     return l;
 }
 
@@ -1306,7 +1287,8 @@ int lensed_set_tuning(lensed* l, const lensed_tuning* t) {
     for (auto& kv : l->layouts) free_layout(l, kv.second);
     l->layouts.clear();
     l->tune_req = req;
-    return build_noalloc_layouts(l);
+    l->noalloc.assign(l->sys.size(), Layout());
+    return 0;
 }
 
 int lensed_autotune_batch(lensed* l, size_t s, size_t* best_k, size_t* ks, double* rates, int* nk) {
@@ -1593,27 +1575,28 @@ int lensed_loglike_batch_noalloc(lensed* l, size_t s, const double* cubes, size_
         set_error("lensed_loglike_batch_noalloc: more candidates than the context's max_batch");
         return -1;
     }
-    Layout& L = l->noalloc[s];
-    lensed_desc& d = L.desc[0];
     // carve the scratch for ncand candidates at 256-byte boundaries
     const size_t nc = ncand;
-    const size_t squares = nc * (size_t)d.ntile_r * (LENSED_RENDER_BS / 64);
+    const size_t squares = nc * (size_t)S.ntile_r * (LENSED_RENDER_BS / 64);
+    const size_t npart = ((S.height + 7) / 8) * ((S.width + LENSED_CONV_TX - 1) / LENSED_CONV_TX);
+    size_t offs[11], total = 0;
     const size_t sizes[] = {sizeof(lensed_desc),
-                            nc * d.npar * 4,
-                            (nc * d.dwords + l->block_pad) * 4,
-                            d.table_mode || S.cull ? nc * LENSED_NPRE_STRIDE(d.table_mode ? d.nq : 0) * 16 : 16,
-                            d.table_mode ? nc * LENSED_EPL_TABLE_F4 * 16 : 16,
-                            nc * (size_t)d.npix * 4,
-                            nc * (size_t)d.npart * 8,
+                            nc * np * 4,
+                            (nc * S.dwords + 256) * 4,
+                            S.table || S.cull ? nc * LENSED_NPRE_STRIDE(S.table ? S.nq : 0) * 16 : 16,
+                            S.table ? nc * LENSED_EPL_TABLE_F4 * 16 : 16,
+                            nc * S.npix * 4,
+                            nc * npart * 8,
                             squares * 4,
-                            live_capacity(squares, nc * ((d.ntile_r + LENSED_CULL_GROUP - 1) / LENSED_CULL_GROUP)) * 4,
+                            live_capacity(squares, nc * ((S.ntile_r + LENSED_CULL_GROUP - 1) / LENSED_CULL_GROUP)) * 4,
                             squares * 4,
                             8};
-    size_t offs[11], total = 0;
     for (int i = 0; i < 11; ++i) {
         offs[i] = total;
         total += (sizes[i] + 255) / 256 * 256;
     }
+    // the words read past the last object block may be those of what follows it
+    total = std::max(total, offs[2] + (nc * S.dwords + l->block_pad) * 4);
     if (total > LENSED_SCRATCH_BYTES) {
         const size_t per = (total - offs[1]) / nc + 1;
         char b[200];
@@ -1639,19 +1622,20 @@ int lensed_loglike_batch_noalloc(lensed* l, size_t s, const double* cubes, size_
     B.owner = (int*)(base + offs[10]);
     B.emulate = false;  // exact-series tables
     B.record = false;   // the context's own statistics are left alone
-    // patch the layout to this call's count
-    const int n = (int)nc;
-    d.ncand = n;
-    L.n_set = L.n_final = n;
-    L.n_render = n * d.ntile_r;
-    L.n_cull = n * ((d.ntile_r + LENSED_CULL_GROUP - 1) / LENSED_CULL_GROUP);
-    L.n_conv = n * (L.conv_rows == LENSED_CONV_SWEEP ? d.tiles_x * d.sweep_seg : d.ntile_c);
-    L.n_table = L.n_nodes = d.table_mode ? n * LENSED_EPL_ROWS : 0;
-    L.n_tcands = d.table_mode ? n : 0;
-    {
-        const double f = L.tune.list_fraction, quads = 16.0 * (double)L.n_render;
-        L.list_max = f < 0 ? 0 : f > 1 ? INT_MAX : (int)std::min<double>(INT_MAX, std::ceil(f * quads));
+    // the launch layout of this count (a single system's offsets into its
+    // buffers are all zero), kept for calls of the same count
+    Layout& L = l->noalloc[s];
+    if (L.n_final != (int)nc) {
+        std::vector<size_t> ncv(l->sys.size(), 0);
+        ncv[s] = nc;
+        L = Layout();
+        if (build_layout(l, ncv, L)) {
+            L = Layout();
+            return -1;
+        }
+        L.id = -2;  // never the id a fill of `owner` leaves (-1)
     }
+    const lensed_desc& d = L.desc[0];
     // parameters into the pinned staging; out-of-bounds draws flagged in lnew_out
     double cube[kMaxPars];
     for (size_t c = 0; c < nc; ++c) {

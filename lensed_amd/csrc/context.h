@@ -184,8 +184,8 @@ struct lensed {
     int next_layout_id = 0;
     unsigned long long layout_clock = 0;
     // the entry point that allocates nothing: this device's static scratch,
-    // a launch layout per system built at creation (patched per call) and a
-    // pinned staging slot for its descriptor
+    // per system the launch layout of the last call's count and a pinned
+    // staging slot for its descriptor
     void* scratch = nullptr;
     std::vector<lsd::Layout> noalloc;
     lensed_desc* h_desc = nullptr;

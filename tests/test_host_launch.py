@@ -31,6 +31,13 @@ def spec(lens, source, shape, psf=None):
     pri = {f"{o}.{p}": "unif 0.5 1" for o, n in (("lens", lens), ("source", source)) for p in params[n].split()}
     return SystemSpec([("lens", lens), ("source", source)], pri, np.zeros(shape, np.float32),
                       np.ones(shape, np.float32), psf=psf)
+
+def noalloc(ctx, n):
+    DP = ctypes.POINTER(ctypes.c_double)
+    cubes, out = np.full((n, ctx.ndims()), 0.5), np.zeros(n)
+    rc = L.load().lensed_loglike_batch_noalloc(ctypes.c_void_p(ctx.ptr), 0, cubes.ctypes.data_as(DP), n, None,
+                                               out.ctypes.data_as(DP))
+    return rc, launches()
 """ % (ROOT, HERE)
 
 
@@ -68,4 +75,26 @@ def test_a_launch_without_candidates_is_an_error(run, lens):
         except LensedError as e:
             assert "no candidates" in str(e)
         assert ctx.loglike_phys([np.zeros((0, ctx.npars(0))), np.full((2, ctx.npars(1)), 0.7)])[1].shape == (2,)
+    """)
+
+
+@pytest.mark.parametrize("lens,source,psf,flags", [("sie", "gauss", 21, 0), ("sie", "sersic", 5, 0),
+                                                   ("epl_plus_shear", "gauss", 21, 4), ("epl_plus_shear", "gauss", 0, 4)])
+def test_the_entry_that_allocates_nothing_launches_as_the_batch(run, lens, source, psf, flags):
+    """For every count the same kernels and grids as lensed_loglike_batch,
+    whatever the context's largest."""
+    run(f"""
+    from lensed_amd import workloads as W
+    with Context(spec({lens!r}, {source!r}, (100, 120), W.gaussian_psf({psf}, 2.0) if {psf} else None), flags={flags},
+                 max_batch=2000) as ctx:
+        seen = set()
+        for n in (2000, 1, 2, 16, 300, 2000, 7):
+            launches()
+            ctx.loglike_batch(np.full((n, ctx.ndims()), 0.5))
+            batch = launches()
+            rc, got = noalloc(ctx, n)
+            assert rc == 0, L.last_error()
+            assert got == batch, (n, got, batch)
+            seen.add(tuple(got))
+        assert len(seen) > 2, seen
     """)

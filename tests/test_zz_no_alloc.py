@@ -68,3 +68,21 @@ def test_noalloc_rejects_what_does_not_fit():
     with Context(wl.spec(), max_batch=8, flags=LENSED_TABLE) as ctx:
         rc, _, _ = noalloc(ctx, np.random.default_rng(8).random((9, ctx.ndims())))
         assert rc == -1 and "max_batch" in L.last_error()
+
+
+# a few candidates under a large max_batch: the small launches' routes (rays
+# shared among waves, no cull pass, a single candidate's partials added up on
+# the host), a sweep in parts, and the large ones again
+@pytest.mark.parametrize("make,flags", [(W.c3, LENSED_TABLE | LENSED_GRAPH), (W.c3, LENSED_GRAPH), (W.c1, 0)])
+def test_noalloc_takes_the_route_of_its_count(make, flags):
+    wl = workload(make)
+    cubes = np.random.default_rng(31).random((400, 20))
+    with Context(wl.spec(), max_batch=400, flags=flags) as ctx:
+        nd = ctx.ndims()
+        for n in (400, 1, 2, 1, 7, 90, 400):
+            ref, pref = ctx.loglike_batch(cubes[:n, :nd])
+            rc, got, pgot = noalloc(ctx, cubes[:n, :nd])
+            assert rc == 0, L.last_error()
+            assert np.all(np.isfinite(got)) and np.array_equal(got, ref) and np.array_equal(pgot, pref), n
+            if n == 1:
+                assert got[0] == ctx.loglike(cubes[0, :nd])[0]
