@@ -294,8 +294,8 @@ static void evict_layouts(::lensed* l) {
 }
 
 // everything of a launch layout but its device descriptors (no allocation
-// on the device); 0 on success
-static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L) {
+// on the device), without a cull pass if cull is false; 0 on success
+static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L, bool cull = true) {
     size_t total = 0;
     for (size_t s = 0; s < l->sys.size(); ++s) {
         if (ncand[s] > l->max_batch) {
@@ -338,7 +338,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
     // dark ones (us of cull and render, with and without the pass, 256 x 256:
     // table 1 candidate 27, 16; 4: 29, 23; 8: 33, 35; series 1: 26, 16; 2: 27,
     // 24; 4: 31, 40)
-    const bool no_cull = (l->flags & LENSED_NO_CULL) || squares < (tables ? 8LL : 3LL) * 4 * l->cu_count;
+    const bool no_cull = !cull || (l->flags & LENSED_NO_CULL) || squares < (tables ? 8LL : 3LL) * 4 * l->cu_count;
     // the column sweep: every system with candidates has a rank-1 separable
     // PSF of at most 21 x 21, and at most 512 rows.  It is the default
     // where every such system is also culled: it skips the rows the cull
@@ -1580,24 +1580,31 @@ int lensed_loglike_batch_noalloc(lensed* l, size_t s, const double* cubes, size_
     const size_t squares = nc * (size_t)S.ntile_r * (LENSED_RENDER_BS / 64);
     const size_t npart = ((S.height + 7) / 8) * ((S.width + LENSED_CONV_TX - 1) / LENSED_CONV_TX);
     size_t offs[11], total = 0;
-    const size_t sizes[] = {sizeof(lensed_desc),
-                            nc * np * 4,
-                            (nc * S.dwords + 256) * 4,
-                            S.table || S.cull ? nc * LENSED_NPRE_STRIDE(S.table ? S.nq : 0) * 16 : 16,
-                            S.table ? nc * LENSED_EPL_TABLE_F4 * 16 : 16,
-                            nc * S.npix * 4,
-                            nc * npart * 8,
-                            squares * 4,
-                            live_capacity(squares, nc * ((S.ntile_r + LENSED_CULL_GROUP - 1) / LENSED_CULL_GROUP)) * 4,
-                            squares * 4,
-                            8};
-    for (int i = 0; i < 11; ++i) {
-        offs[i] = total;
-        total += (sizes[i] + 255) / 256 * 256;
-    }
-    // the words read past the last object block may be those of what follows it
-    total = std::max(total, offs[2] + (nc * S.dwords + l->block_pad) * 4);
-    if (total > LENSED_SCRATCH_BYTES) {
+    auto carve = [&](bool cull) {
+        const size_t sizes[] = {sizeof(lensed_desc),
+                                nc * np * 4,
+                                (nc * S.dwords + 256) * 4,
+                                S.table || cull ? nc * LENSED_NPRE_STRIDE(S.table ? S.nq : 0) * 16 : 16,
+                                S.table ? nc * LENSED_EPL_TABLE_F4 * 16 : 16,
+                                nc * S.npix * 4,
+                                nc * npart * 8,
+                                squares * 4,
+                                live_capacity(squares, nc * ((S.ntile_r + LENSED_CULL_GROUP - 1) / LENSED_CULL_GROUP)) * 4,
+                                squares * 4,
+                                8};
+        total = 0;
+        for (int i = 0; i < 11; ++i) {
+            offs[i] = total;
+            total += (sizes[i] + 255) / 256 * 256;
+        }
+        // the words read past the last object block may be those of what follows it
+        total = std::max(total, offs[2] + (nc * S.dwords + l->block_pad) * 4);
+        return total <= LENSED_SCRATCH_BYTES;
+    };
+    // a system without a table does without the cull where its constants
+    // would be what does not fit
+    const bool cull = carve(S.cull);
+    if (!cull && (S.table || !S.cull || !carve(false))) {
         const size_t per = (total - offs[1]) / nc + 1;
         char b[200];
         snprintf(b, sizeof b,
@@ -1629,7 +1636,7 @@ int lensed_loglike_batch_noalloc(lensed* l, size_t s, const double* cubes, size_
         std::vector<size_t> ncv(l->sys.size(), 0);
         ncv[s] = nc;
         L = Layout();
-        if (build_layout(l, ncv, L)) {
+        if (build_layout(l, ncv, L, cull)) {
             L = Layout();
             return -1;
         }

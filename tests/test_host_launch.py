@@ -98,3 +98,31 @@ def test_the_entry_that_allocates_nothing_launches_as_the_batch(run, lens, sourc
             seen.add(tuple(got))
         assert len(seen) > 2, seen
     """)
+
+
+@pytest.mark.parametrize("shape", [(16, 16), (40, 24), (64, 100)])
+def test_scratch_holds_as_many_candidates_with_the_cull(run, shape):
+    """Culled without a table: the cull's constants do not push a count out
+    of the scratch that fits it without them."""
+    run(f"""
+    h, w = {shape}
+    s = spec("sie", "gauss", (h, w))
+    words, npar = sum(o.obj.size for o in s.objects), sum(o.obj.npars for o in s.objects)
+    items = -(-h // 16) * -(-w // 16)
+    up = lambda n: -(-n // 256) * 256
+    def need(n):  # descriptor, parameters, blocks, two unused, model, partials, flags, list, record, owner
+        parts = [512, n * npar * 4, (n * words + 256) * 4, 16, 16, n * h * w * 4, n * -(-h // 8) * -(-w // 64) * 8,
+                 n * items * 16, 4 * (1 + 16 * n * items + 16 * n * -(-items // 64)), n * items * 16, 8]
+        return sum(up(p) for p in parts)
+    n = max(k for k in range(1, 110000) if need(k) <= 128 << 20) if h * w < 300 else (128 << 20) // (need(1000) // 1000)
+    while need(n) > 128 << 20:
+        n -= 1
+    with Context(s, max_batch=n + n // 8) as ctx:
+        rc, got = noalloc(ctx, n)
+        assert rc == 0, L.last_error()
+        assert "lensed_cull" not in got, got
+        rc, got = noalloc(ctx, n - n // 8)
+        assert rc == 0 and "lensed_cull" in got, (L.last_error(), got)
+        rc, got = noalloc(ctx, n + n // 8)
+        assert rc != 0 and "static scratch" in L.last_error() and not got
+    """)

@@ -12,7 +12,7 @@ import pytest
 from lensed_amd import _lib as L
 from lensed_amd import workloads as W
 from lensed_amd._lib import LENSED_GRAPH, LENSED_TABLE
-from lensed_amd.lensed import Context
+from lensed_amd.lensed import Context, SystemSpec
 from oracle import oracle as O
 from test_gpu_parity import oracle_render_cb
 
@@ -86,3 +86,26 @@ def test_noalloc_takes_the_route_of_its_count(make, flags):
             assert np.all(np.isfinite(got)) and np.array_equal(got, ref) and np.array_equal(pgot, pref), n
             if n == 1:
                 assert got[0] == ctx.loglike(cubes[0, :nd])[0]
+
+
+def test_noalloc_without_the_cull_at_the_scratch_limit():
+    """A count that fits the scratch only without the cull's constants."""
+    shape = (16, 16)
+    span = {"lens.x": "unif 7 10", "lens.y": "unif 7 10", "lens.r": "unif 2 4", "lens.q": "unif 0.5 0.9",
+            "lens.pa": "unif 0 180", "s.x": "unif 7 10", "s.y": "unif 7 10", "s.sigma": "unif 0.1 0.3",
+            "s.mag": "unif -3 3", "s.q": "unif 0.5 1", "s.pa": "unif 0 180"}
+    rng = np.random.default_rng(41)
+    spec = SystemSpec([("lens", "sie"), ("s", "gauss")], span, rng.normal(0, 0.05, shape).astype(np.float32),
+                      np.full(shape, 400.0, np.float32))
+    cubes = rng.random((110000, len(span)))
+    with Context(spec, max_batch=110000, flags=LENSED_GRAPH) as ctx:
+        ref, _ = ctx.loglike_batch(cubes)
+        counts = []
+        n = 110000
+        while n > 80000:  # steps of 500, well under the 3 % that the constants take
+            rc, got, _ = noalloc(ctx, cubes[:n])
+            if rc == 0:
+                assert np.array_equal(got, ref[:n]), n
+                counts.append(n)
+            n -= 500 if not counts else 5000
+        assert len(counts) >= 2, counts
