@@ -426,9 +426,12 @@ std::string compute_function(const std::vector<ModelObject>& objs, int k) {
     // where it was (the same number in FP32 within 512 pixels of the origin,
     // 1024 pixels apart at most steps further out, and no source's light
     // either way): the subtraction then stands between the comparison and the
-    // selects that wait for it.
+    // selects that wait for it.  The deflection is rounded first, so that the
+    // subtraction and a product at the deflection's end (sis, nsis,
+    // point_mass) stay two operations.
     auto close_plane = [&]() {
-        o << "        const float2 r = " << (lin ? "float2(pre.z, pre.w)" : "y") << " - a;\n"
+        o << "        a = lensed_rounded(a);\n"
+          << "        const float2 r = " << (lin ? "float2(pre.z, pre.w)" : "y") << " - a;\n"
           << "        y = lensed_deflection_ok(a) ? r : float2(-1E10f, -1E10f);\n    }\n";
         plane_open = false;
     };

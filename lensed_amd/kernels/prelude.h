@@ -258,6 +258,17 @@ inline void lensed_branch() {
 #endif
 }
 
+// A value rounded before it is used: what follows does not take the product
+// behind it into a fused multiply-add.  (A statement per component: one for
+// both holds back the first until the second is there.)
+inline float2 lensed_rounded(float2 a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(a.x));
+    asm("" : "+v"(a.y));
+#endif
+    return a;
+}
+
 // ---------------------------------------------------------------- geometry
 inline float dot(float2 a, float2 b) { return a.x * b.x + a.y * b.y; }
 inline float dot(float4 a, float4 b) { return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w; }
