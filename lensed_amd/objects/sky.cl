@@ -23,7 +23,7 @@ static float foreground(local data* this, float2 x)
     if(this->grad.x != 0 || this->grad.y != 0)
     {
         lensed_branch();
-        f += dot(this->grad, x - (float2)(1, 1));
+        f += fma(this->grad.x, x.x - 1, this->grad.y*(x.y - 1));
     }
     return f;
 }

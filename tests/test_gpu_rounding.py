@@ -1,10 +1,11 @@
-"""A deflection is rounded to FP32 before it is subtracted from the ray's
-position: a lens whose deflection ends in a product, and a source that gives
-the ray's x, against the two operations in numpy."""
+"""Which products the ray loop fuses with the sum that follows, against the
+same operations one by one on the host: logL has the bits of these pairings."""
+from fractions import Fraction
+
 import numpy as np
 import pytest
 
-from lensed_amd._lib import LENSED_GRAPH
+from lensed_amd._lib import LENSED_GRAPH, LENSED_TABLE
 from lensed_amd.lensed import Context, SystemSpec
 
 pytestmark = pytest.mark.gpu
@@ -23,6 +24,12 @@ static void set(local data* this, float s) { this->s = s; }
 """
 
 
+def fma(a, b, c):
+    return np.float32(float(Fraction(float(a)) * Fraction(float(b)) + Fraction(float(c))))
+
+
+# a lens whose deflection ends in a product, and a source that gives the ray's
+# position: the deflection is rounded before it is subtracted
 @pytest.mark.parametrize("axis", ["x", "y"])
 @pytest.mark.parametrize("n", [1, 40, 3000])  # a wave per 64 pixels and rays shared
 def test_deflection_is_rounded_before_the_subtraction(tmp_path, monkeypatch, axis, n):
@@ -48,3 +55,26 @@ def test_deflection_is_rounded_before_the_subtraction(tmp_path, monkeypatch, axi
             logl = ctx.loglike_phys(phys)
             ref = -0.5 * np.sum((want * want).astype(np.float64))
             assert np.all(np.abs(logl - ref) <= 512 * 2.0 ** -47 * abs(ref)), k
+
+
+# a sky with a gradient behind nothing, a lens and a tabulated lens (dark
+# sources: what they add is 0): level + fma(gx, x - 1, gy (y - 1)), and the
+# level alone without a gradient
+@pytest.mark.parametrize("objects,flags", [(["sky"], 0), (["sie", "sersic", "sky"], 0), (["epl", "sersic", "sky"], LENSED_TABLE),
+                                           (["epl_plus_shear", "gauss", "gauss", "sky"], LENSED_TABLE)])
+@pytest.mark.parametrize("grad", [(0.0, 0.0), (1.3e-3, -7.7e-4), (0.0, 3.1e-4)])
+def test_sky_gradient_is_one_fma(objects, flags, grad):
+    shape, level = (33, 50), np.float32(0.0173)
+    gx, gy = np.float32(grad)
+    values = {"x": 25.2, "y": 16.4, "r": 5.0, "t": 1.1, "q": 0.7, "pa": 40.0, "g1": 0.02, "g2": -0.03, "sigma": 0.01,
+              "n": 1.0, "mag": 400.0, "bg": float(level), "dx": float(gx), "dy": float(gy)}
+    params = {"sky": "bg dx dy", "sie": "x y r q pa", "epl": "x y r t q pa", "epl_plus_shear": "x y r t q pa g1 g2",
+              "sersic": "x y r mag n q pa", "gauss": "x y sigma mag q pa"}
+    pri = {f"o{i}.{p}": repr(values[p]) for i, n in enumerate(objects) for p in params[n].split()}
+    spec = SystemSpec([(f"o{i}", n) for i, n in enumerate(objects)], pri, np.zeros(shape, np.float32),
+                      np.ones(shape, np.float32), rule="point")
+    with Context(spec, flags=flags) as ctx:
+        got = ctx.render([values[p] for n in objects for p in params[n].split()])["value"]
+    want = np.array([[level + fma(gx, np.float32(j), gy * np.float32(i)) for j in range(shape[1])]
+                     for i in range(shape[0])], np.float32)
+    assert np.array_equal(got, want)
