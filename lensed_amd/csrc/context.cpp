@@ -60,8 +60,9 @@ std::string model_source(const std::vector<std::vector<ModelObject>>& models, st
         if (po != std::string::npos) t->erase(po, 12);
     }
     std::ostringstream o;
-    o << "// generated by lensed-amd: prelude, objects, model code\n"
-      << prelude << "\n" << desc
+    o << "// generated by lensed-amd: prelude, objects, model code\n";
+    if (std::any_of(models.begin(), models.end(), model_adds_exps)) o << "#define LCL_PLAIN_EXP\n";
+    o << prelude << "\n" << desc
       << "\n#ifdef LCL_GPU\n#pragma clang force_cuda_host_device begin\n#endif\nnamespace lcl {\n";
     std::set<std::string> seen;
     for (const auto& m : models)

@@ -361,6 +361,12 @@ static bool slope_culls(const std::vector<ModelObject>& objs) {
     return true;
 }
 
+bool model_adds_exps(const std::vector<ModelObject>& objs) {
+    int n = 0;
+    for (const auto& ob : objs) n += ob.type == OBJ_SOURCE && plugin_defines(ob.name, {R"(\bexp\s*\()"});
+    return n > 1;
+}
+
 bool model_holds(const std::vector<ModelObject>& objs) {
     // at most 64 words, so that the block and the ray's own values (about 50
     // registers with two sources) stay within the loop's 128 registers

@@ -66,6 +66,8 @@ std::string compute_function(const std::vector<ModelObject>& objs, int k);
 // EPL lens and one source with a frame and a cutoff, nothing else; or lenses
 // that bound their own slope (deflection_slope), then compact sources
 bool model_culls(const std::vector<ModelObject>& objs);
+// whether several of the model's sources use exp()
+bool model_adds_exps(const std::vector<ModelObject>& objs);
 // whether the render holds the model's data block in vector registers
 bool model_holds(const std::vector<ModelObject>& objs);
 std::string set_params_function(const std::vector<ModelObject>& objs, int k);

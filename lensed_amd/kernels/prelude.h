@@ -185,7 +185,11 @@ LCL_TRANS(lensed_sqrt, "v_sqrt_f32", ::sqrtf)
 #undef LCL_TRANS
 #undef LCL_RECIP_FIRST
 #undef LCL_F1
-#if defined(__HIP_DEVICE_COMPILE__)
+// (LCL_PLAIN_EXP: set where a model adds up several sources that end in a
+// product with exp().  The compiler fuses one of the first two products with
+// the sum, by the depth of what is behind them, and takes an inline statement
+// for deeper than everything before it.)
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(LCL_PLAIN_EXP)
 inline float exp(float a) { return exp2(a * 1.44269504088896340736f); }
 #else
 inline float exp(float a) { return ::expf(a); }

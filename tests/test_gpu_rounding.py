@@ -78,3 +78,41 @@ def test_sky_gradient_is_one_fma(objects, flags, grad):
     want = np.array([[level + fma(gx, np.float32(j), gy * np.float32(i)) for j in range(shape[1])]
                      for i in range(shape[0])], np.float32)
     assert np.array_equal(got, want)
+
+
+PRODUCT = """type = SOURCE;
+params { { "x", POSITION_X }, { "y", POSITION_Y }, { "s", PARAMETER } };
+data { float2 c; float s; };
+static float brightness(local data* this, float2 x) { return this->s*exp(%s); }
+static void set(local data* this, float x, float y, float s) { this->c = (float2)(x, y); this->s = s; }
+"""
+
+
+# two products with exp(), the first behind a longer chain: the second product
+# is fused with the sum in either order, the first is rounded (each exponential
+# is read off with a factor of 1)
+@pytest.mark.parametrize("lens", ["sis", "sie"])
+@pytest.mark.parametrize("order", ["deep shallow", "shallow deep"])
+def test_the_shallower_of_two_products_is_fused(tmp_path, monkeypatch, lens, order):
+    (tmp_path / "deep.cl").write_text(PRODUCT % "-3.3f*sqrt(sqrt(length(x - this->c)/7))")
+    (tmp_path / "shallow.cl").write_text(PRODUCT % "-length(x - this->c)/9")
+    monkeypatch.setenv("LENSED_OBJECTS_PATH", str(tmp_path))
+    shape = (33, 50)
+    values = {"x": 25.3, "y": 16.4, "r": 5.0, "q": 0.7, "pa": 40.0}
+    lp = {"sis": "x y r", "sie": "x y r q pa"}[lens].split()
+    names = order.split()
+    pri = {f"l.{p}": repr(values[p]) for p in lp}
+    pri.update({f"{n}.{p}": "unif 0 60" for n in names for p in ("x", "y", "s")})
+    spec = SystemSpec([("l", lens)] + [(n, n) for n in names], pri, np.zeros(shape, np.float32),
+                      np.ones(shape, np.float32), rule="point")
+    centre = {"deep": (20.1, 18.2), "shallow": (27.7, 13.9)}
+    with Context(spec) as ctx:
+        def value(**s):
+            return ctx.render([values[p] for p in lp] + [v for n in names for v in (*centre[n], s.get(n, 0.0))])["value"]
+        e = {n: value(**{n: 1.0}) for n in names}
+        for s in (0.37, 1.7):
+            s = {"deep": np.float32(s), "shallow": np.float32(1 / s)}
+            got = value(**s)
+            want = [[fma(s["shallow"], e["shallow"][i, j], s["deep"] * e["deep"][i, j]) for j in range(shape[1])]
+                    for i in range(shape[0])]
+            assert np.array_equal(got, np.array(want, np.float32)), s
