@@ -257,7 +257,8 @@ typedef struct {
     double cull_grid;     /* pixel-cull blocks, the same (4) */
     double conv_grid;     /* convolution blocks, the same (1) */
     int conv_rows;        /* output rows per thread of the convolution tile (4 rows of threads): 2, 8 or 16
-                             (the largest with two tiles per compute unit); 16 needs 64 + PSF
+                             (the launch has enough tiles for each compute unit, and for 16 the images
+                             hold whole tiles with little left over); 16 needs 64 + PSF
                              height - 1 rows of LDS and falls back to 8 where that passes 64 KiB; or 1, the
                              column sweep: one wave per 64-column strip of an image runs down the strip,
                              for launches whose systems all have a rank-1 separable PSF of at most 21 x 21 and

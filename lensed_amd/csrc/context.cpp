@@ -309,25 +309,45 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
         set_error("no candidates");
         return -1;
     }
-    // conv tile height: the tallest of which the launch has two per CU.  (us,
-    // 8-, 32- and 64-row tiles, by the number of 64-row ones: direct 31 x 31
-    // taps 256: 46, 41, 47; 512: 84, 66, 52; 32768: 4782, 3782, 2750; two
-    // passes of 21 taps 256: 12, 11, 12; 512: 18, 13.0, 13.6; 1024: 30, 17.5,
-    // 16.7; 16384: 366, 204, 177)
-    auto tiles = [&](int rows) {
-        long long n = 0;
-        for (size_t s = 0; s < l->sys.size(); ++s) {
-            const System& S = l->sys[s];
-            n += (long long)ncand[s] * ((S.width + LENSED_CONV_TX - 1) / LENSED_CONV_TX) *
-                 ((S.height + LENSED_CONV_TY * rows - 1) / (LENSED_CONV_TY * rows));
+    // conv tile height: 32 rows where the launch has two such tiles per CU,
+    // and 64 where it has enough of those and rounding the images up to whole
+    // tiles adds little.  (us, 8-, 32- and 64-row tiles, by the number of
+    // 64-row ones.  Images of 64 rows: direct 31 x 31 taps 256: 46, 41, 47;
+    // 512: 77, 65, 53; 8192: 1162, 941, 694; row and column passes, 21 x 21
+    // taps 512: 18.6, 12.8, 12.6; 16384: 445, 232, 182; 22 x 8 taps 600: 17.6,
+    // 12.7, 13.7; 7 x 7 taps 600: 16, 10.6, 11.5; 768: 20, 11.7, 11.7; 16384:
+    // 344, 163, 134; no PSF 768: 13.4, 8.2, 8.8; 1024: 16, 9.6, 9.3; 16384:
+    // 196, 86, 68.  Of 32, half a tall tile, 4096: 31 x 31 322, 235, 344; 7 x 7
+    // 49, 24, 35.  Of 80, a third more in tall tiles, 8192: 719, 710, 685 and
+    // 108, 60, 67.  Of 160, a fifth more, 8192: 966, 797, 686 and 144, 69, 68;
+    // 13 x 13 taps 16384: 335, 144, 149.  Images of at most four rows don't
+    // count, what they fill of a tile of either height is next to nothing:
+    // 600 of 1 x 70, 3 x 3 taps: 7.7, 9.5, 12.1)
+    long long n32 = 0, n64 = 0, r32 = 0, r64 = 0;
+    long long per_cu = 2;  // tall tiles the launch has to have
+    double grown = 1.4;    // rows in tall tiles to rows in 32-row ones, below this
+    for (size_t s = 0; s < l->sys.size(); ++s) {
+        const System& S = l->sys[s];
+        if (!ncand[s]) continue;
+        auto tiles = [&](size_t rows) {
+            return (long long)(ncand[s] * ((S.width + LENSED_CONV_TX - 1) / LENSED_CONV_TX) *
+                               ((S.height + LENSED_CONV_TY * rows - 1) / (LENSED_CONV_TY * rows)));
+        };
+        const long long t32 = tiles(LENSED_CONV_RY), t64 = tiles(LENSED_CONV_RY_TALL);
+        const size_t taps = S.psfw * S.psfh;
+        n32 += t32;
+        n64 += t64;
+        if (S.height > LENSED_CONV_TY) {
+            r32 += t32 * LENSED_CONV_RY;
+            r64 += t64 * LENSED_CONV_RY_TALL;
+            grown = std::min(grown, taps >= 600 && !S.sep_rank ? 1.4 : taps >= 170 || !taps ? 1.25 : 1.2);
         }
-        return n;
-    };
-    L.conv_small = tiles(LENSED_CONV_RY) < 2LL * l->cu_count;
+        per_cu = std::max(per_cu, taps >= 170 ? 2LL : taps ? 3LL : 4LL);
+    }
+    L.conv_small = n32 < 2LL * l->cu_count;
     const lensed_tuning& tq = l->tune_req;
-    const int rows_default = L.conv_small                                       ? LENSED_CONV_RY_SMALL
-                             : tiles(LENSED_CONV_RY_TALL) < 2LL * l->cu_count ? LENSED_CONV_RY
-                                                                              : LENSED_CONV_RY_TALL;
+    const bool tall = n64 >= per_cu * l->cu_count && (!r32 || (double)r64 < grown * (double)r32);
+    const int rows_default = L.conv_small ? LENSED_CONV_RY_SMALL : tall ? LENSED_CONV_RY_TALL : LENSED_CONV_RY;
     L.conv_rows = tq.conv_rows ? tq.conv_rows : rows_default;
     long long squares = 0;  // 64 pixels each: a wave of the render
     bool tables = false;

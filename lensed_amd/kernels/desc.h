@@ -11,7 +11,7 @@
 #define LENSED_CONV_TY 4      // threads along y
 #define LENSED_CONV_RY 8      // output rows per thread, large launches (a multiple of 8)
 #define LENSED_CONV_RY_SMALL 2  // output rows per thread, launches too small to fill the GPU
-#define LENSED_CONV_RY_TALL 16  // output rows per thread of the 64-row tile (a tuning choice)
+#define LENSED_CONV_RY_TALL 16  // output rows per thread of the 64-row tile (large launches of images that fill it)
 #define LENSED_CONV_SWEEP 1   // conv_rows value of the column sweep: one wave per 64-column strip
 #define LENSED_SWEEP_MAX_H 512  // the sweep's 8-row band flags fit one 64-bit mask
 #define LENSED_SWEEP_MAX_PSF 21  // the sweep's PSF sides at most: its PH-row window is unrolled, and its

@@ -126,3 +126,25 @@ def test_scratch_holds_as_many_candidates_with_the_cull(run, shape):
         rc, got = noalloc(ctx, n + n // 8)
         assert rc != 0 and "static scratch" in L.last_error() and not got
     """)
+
+
+@pytest.mark.parametrize("psf", [0, 7, 13, 31])
+def test_tall_tiles_only_where_the_images_fill_them(run, psf):
+    """64-row tiles for images whose rows they hold with little left over,
+    whatever the number of candidates."""
+    run(f"""
+    from lensed_amd import workloads as W
+    def kernel(h, n):
+        with Context(spec("sie", "sersic", (h, 64), W.moffat_psf({psf}, 3.0, 2.5) if {psf} else None), max_batch=n) as ctx:
+            launches()
+            ctx.loglike_batch(np.full((n, ctx.ndims()), 0.5))
+            return next(k for k in launches() if k.startswith("lensed_conv"))
+    for h in (5, 20, 32, 65, 80, 96):
+        tall = h > 32 and {psf} == 31  # (direct)
+        assert kernel(h, 8192) == "lensed_conv_chi2" + ("_tall" if tall else ""), h
+    for h in (33, 64, 97, 128, 200, 256):
+        assert kernel(h, 4096) == "lensed_conv_chi2_tall", h
+    assert kernel(160, 4096) == ("lensed_conv_chi2" if {psf} in (7, 13) else "lensed_conv_chi2_tall")
+    assert kernel(64, 600) == ("lensed_conv_chi2_tall" if {psf} > 14 else "lensed_conv_chi2")
+    assert kernel(64, 100) == "lensed_conv_chi2_small"
+    """)
