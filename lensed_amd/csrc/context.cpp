@@ -350,16 +350,22 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
     const int rows_default = L.conv_small ? LENSED_CONV_RY_SMALL : tall ? LENSED_CONV_RY_TALL : LENSED_CONV_RY;
     L.conv_rows = tq.conv_rows ? tq.conv_rows : rows_default;
     long long squares = 0;  // 64 pixels each: a wave of the render
-    bool tables = false;
+    bool tables = false, series = false;
     for (size_t s = 0; s < l->sys.size(); ++s) {
         squares += 4LL * (long long)ncand[s] * l->sys[s].ntile_r;
         tables = tables || (ncand[s] && l->sys[s].table);
+        series = series || (ncand[s] && l->sys[s].series);
     }
     // no cull pass where tracing every ray takes no longer than finding the
     // dark ones (us of cull and render, with and without the pass, 256 x 256:
     // table 1 candidate 27, 16; 4: 29, 23; 8: 33, 35; series 1: 26, 16; 2: 27,
-    // 24; 4: 31, 40)
-    const bool no_cull = !cull || (l->flags & LENSED_NO_CULL) || squares < (tables ? 8LL : 3LL) * 4 * l->cu_count;
+    // 24; 4: 31, 40.  Whole calls with Gaussians of 1/8 of the Einstein radius,
+    // by the number of squares, EPL + shear by its series 128 x 128 3072: 72,
+    // 53; 4096: 70, 59; 160 x 160 6000: 81, 80; 8400: 92, 97; SIE 128 x 128
+    // 3072: 72, 69; 256 x 256 4096: 71, 76; 200 x 200 4056: 75, 95)
+    const long long fill = 4LL * l->cu_count;  // one square per SIMD
+    const bool no_cull = !cull || (l->flags & LENSED_NO_CULL) ||
+                         (tables ? squares < 8 * fill : series ? squares <= 4 * fill : squares < 3 * fill);
     // the column sweep: every system with candidates has a rank-1 separable
     // PSF of at most 21 x 21, and at most 512 rows.  It is the default
     // where every such system is also culled: it skips the rows the cull
@@ -1072,6 +1078,17 @@ lensed* lensed_create(const lensed_system* systems, size_t nsys, const lensed_op
         S.sigma.assign(np, 0);
         S.ml.assign(np, 0);
         S.map.assign(np, 0);
+        // images of a few blocks are lit nearly throughout, a Gaussian's
+        // cutoff being 13 sigma out, and a series lens (whose rays cost half
+        // an SIE's, its bound as much again) gains nothing there.  (us a call,
+        // culled and not, without a table, sigma 1/8 of the Einstein radius:
+        // EPL + shear 16 x 16 4375 candidates 273, 223; 24 x 24 1500: 170,
+        // 150; 32 x 32 262: 90, 74; 40 x 40 1333: 230, 288; SIE 16 x 16 4375:
+        // 345, 300; 24 x 24 262: 86, 98; 32 x 32 193: 94, 97; 3000: 569, 539)
+        if (S.cull && !S.table) {
+            for (const auto& ob : S.objs) S.series = S.series || (ob.type == OBJ_LENS && object_tabulates(ob.name));
+            if (S.ntile_r < (S.series ? 9 : 4)) S.cull = false;
+        }
         l->sys.push_back(S);
     }
     if (psf.empty()) psf.push_back(0.0f);

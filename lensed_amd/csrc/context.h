@@ -64,6 +64,7 @@ struct System {
     // dumper results (object order)
     std::vector<double> mean, sigma, ml, map;
     double logev = 0, logev_err = 0, logev_ins = 0, max_loglike = 0;
+    bool series = false;  // a lens of the model sums its angular series for each ray
     // the candidates of the last lensed_loglike_batch() call whose EPL table
     // the emulator built (1) rather than the exact series (0); empty when
     // no table came from the network

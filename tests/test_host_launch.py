@@ -100,7 +100,7 @@ def test_the_entry_that_allocates_nothing_launches_as_the_batch(run, lens, sourc
     """)
 
 
-@pytest.mark.parametrize("shape", [(16, 16), (40, 24), (64, 100)])
+@pytest.mark.parametrize("shape", [(48, 48), (40, 72), (64, 100)])
 def test_scratch_holds_as_many_candidates_with_the_cull(run, shape):
     """Culled without a table: the cull's constants do not push a count out
     of the scratch that fits it without them."""
@@ -114,7 +114,7 @@ def test_scratch_holds_as_many_candidates_with_the_cull(run, shape):
         parts = [512, n * npar * 4, (n * words + 256) * 4, 16, 16, n * h * w * 4, n * -(-h // 8) * -(-w // 64) * 8,
                  n * items * 16, 4 * (1 + 16 * n * items + 16 * n * -(-items // 64)), n * items * 16, 8]
         return sum(up(p) for p in parts)
-    n = max(k for k in range(1, 110000) if need(k) <= 128 << 20) if h * w < 300 else (128 << 20) // (need(1000) // 1000)
+    n = (128 << 20) // (need(1000) // 1000)
     while need(n) > 128 << 20:
         n -= 1
     with Context(s, max_batch=n + n // 8) as ctx:
@@ -147,4 +147,20 @@ def test_tall_tiles_only_where_the_images_fill_them(run, psf):
     assert kernel(160, 4096) == ("lensed_conv_chi2" if {psf} in (7, 13) else "lensed_conv_chi2_tall")
     assert kernel(64, 600) == ("lensed_conv_chi2_tall" if {psf} > 14 else "lensed_conv_chi2")
     assert kernel(64, 100) == "lensed_conv_chi2_small"
+    """)
+
+
+def test_cull_pass_only_where_it_can_skip_enough(run):
+    """Without a table: by squares of 64 pixels per SIMD, and not for images of
+    a few 16 x 16 blocks."""
+    run("""
+    def culled(lens, shape, n):
+        with Context(spec(lens, "gauss", shape), max_batch=n) as ctx:
+            launches()
+            ctx.loglike_batch(np.full((n, ctx.ndims()), 0.5))
+            return "lensed_cull" in launches()
+    assert not culled("epl_plus_shear", (128, 128), 16) and culled("epl_plus_shear", (128, 128), 17)
+    assert not culled("sie", (128, 128), 11) and culled("sie", (128, 128), 12)
+    assert not culled("epl_plus_shear", (32, 32), 4000) and culled("epl_plus_shear", (40, 40), 4000)
+    assert not culled("sie", (16, 48), 4000) and culled("sie", (24, 24), 4000)
     """)

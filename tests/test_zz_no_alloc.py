@@ -90,22 +90,22 @@ def test_noalloc_takes_the_route_of_its_count(make, flags):
 
 def test_noalloc_without_the_cull_at_the_scratch_limit():
     """A count that fits the scratch only without the cull's constants."""
-    shape = (16, 16)
-    span = {"lens.x": "unif 7 10", "lens.y": "unif 7 10", "lens.r": "unif 2 4", "lens.q": "unif 0.5 0.9",
-            "lens.pa": "unif 0 180", "s.x": "unif 7 10", "s.y": "unif 7 10", "s.sigma": "unif 0.1 0.3",
+    shape = (48, 48)
+    span = {"lens.x": "unif 23 26", "lens.y": "unif 23 26", "lens.r": "unif 4 7", "lens.q": "unif 0.5 0.9",
+            "lens.pa": "unif 0 180", "s.x": "unif 23 26", "s.y": "unif 23 26", "s.sigma": "unif 0.1 0.3",
             "s.mag": "unif -3 3", "s.q": "unif 0.5 1", "s.pa": "unif 0 180"}
     rng = np.random.default_rng(41)
     spec = SystemSpec([("lens", "sie"), ("s", "gauss")], span, rng.normal(0, 0.05, shape).astype(np.float32),
                       np.full(shape, 400.0, np.float32))
-    cubes = rng.random((110000, len(span)))
-    with Context(spec, max_batch=110000, flags=LENSED_GRAPH) as ctx:
+    cubes = rng.random((14500, len(span)))
+    with Context(spec, max_batch=14500, flags=LENSED_GRAPH) as ctx:
         ref, _ = ctx.loglike_batch(cubes)
         counts = []
-        n = 110000
-        while n > 80000:  # steps of 500, well under the 3 % that the constants take
+        n = 14500
+        while n > 12000:  # steps of 20, under the 0.5 % that the constants take
             rc, got, _ = noalloc(ctx, cubes[:n])
             if rc == 0:
                 assert np.array_equal(got, ref[:n]), n
                 counts.append(n)
-            n -= 500 if not counts else 5000
+            n -= 20 if not counts else 500
         assert len(counts) >= 2, counts
