@@ -16,6 +16,7 @@
 #include <sys/stat.h>
 
 #include <algorithm>
+#include <cctype>
 #include <cstdio>
 #include <cstdlib>
 #include <fstream>
@@ -326,6 +327,38 @@ static int frame_source(const std::vector<ModelObject>& objs) {
     return src;
 }
 
+// whether every return of the lens's deflection() is a sum of matrices times
+// vectors, mv22(...) [+- mv22(...)]: a sum at its end, which no subtraction
+// fuses with
+static bool ends_in_sum(const std::string& name) {
+    const std::string src = without_comments(plugin_text(name));
+    std::smatch m;
+    if (!std::regex_search(src, m, std::regex(R"(static\s+float2\s+deflection\s*\()"))) return false;
+    const size_t b = m.position(0), e = src.find("\n}", b);
+    const std::string body = src.substr(b, e == std::string::npos ? e : e - b);
+    auto blank = [&](size_t& i) { while (i < body.size() && isspace((unsigned char)body[i])) ++i; };
+    int n = 0;
+    for (size_t i = body.find("return"); i != std::string::npos; i = body.find("return", i), ++n) {
+        i += 6;
+        for (;;) {
+            blank(i);
+            if (body.compare(i, 4, "mv22") != 0) return false;
+            blank(i += 4);
+            if (i >= body.size() || body[i] != '(') return false;
+            for (int depth = 0; i < body.size(); ++i) {
+                depth += body[i] == '(' ? 1 : body[i] == ')' ? -1 : 0;
+                if (depth == 0) break;
+            }
+            if (i >= body.size()) return false;
+            blank(++i);
+            if (i < body.size() && body[i] == ';') break;
+            if (i >= body.size() || (body[i] != '+' && body[i] != '-')) return false;
+            ++i;
+        }
+    }
+    return n > 0;
+}
+
 // The lens-frame cull: the tabulated lens and its framed source alone, so a
 // skipped pixel's value is exactly 0.
 static bool frame_culls(const std::vector<ModelObject>& objs) {
@@ -434,10 +467,14 @@ std::string compute_function(const std::vector<ModelObject>& objs, int k) {
     // either way): the subtraction then stands between the comparison and the
     // selects that wait for it.  The deflection is rounded first, so that the
     // subtraction and a product at the deflection's end (sis, nsis,
-    // point_mass) stay two operations.
+    // point_mass) stay two operations; one that ends in a sum needs no help
+    // (2048 candidates of 100 x 100, SIE + Gaussian: 1613 us without it, 1642
+    // with).
+    bool round = false;
+    for (const auto& ob : objs) round = round || (ob.type == OBJ_LENS && !ob.table && !ends_in_sum(ob.name));
     auto close_plane = [&]() {
-        o << "        a = lensed_rounded(a);\n"
-          << "        const float2 r = " << (lin ? "float2(pre.z, pre.w)" : "y") << " - a;\n"
+        if (round) o << "        a = lensed_rounded(a);\n";
+        o << "        const float2 r = " << (lin ? "float2(pre.z, pre.w)" : "y") << " - a;\n"
           << "        y = lensed_deflection_ok(a) ? r : float2(-1E10f, -1E10f);\n    }\n";
         plane_open = false;
     };

@@ -13,7 +13,10 @@ pytestmark = pytest.mark.gpu
 LENS = """type = LENS;
 params { { "x", POSITION_X }, { "y", POSITION_Y }, { "k", PARAMETER } };
 data { float2 c; float k; };
-static float2 deflection(local data* this, float2 x) { return this->k*(x - this->c); }
+static float2 deflection(local data* this, float2 x)
+{
+    return %s;
+}
 static void set(local data* this, float x, float y, float k) { this->c = (float2)(x, y); this->k = k; }
 """
 SOURCE = """type = SOURCE;
@@ -31,9 +34,11 @@ def fma(a, b, c):
 # a lens whose deflection ends in a product, and a source that gives the ray's
 # position: the deflection is rounded before it is subtracted
 @pytest.mark.parametrize("axis", ["x", "y"])
+@pytest.mark.parametrize("form", ["this->k*(x - this->c)", "mv22((mat22)(1, 0, 0, 1), x - this->c)*this->k",
+                                  "mv22((mat22)(1, 0, 0, 1), this->k*(x - this->c))"])
 @pytest.mark.parametrize("n", [1, 40, 3000])  # a wave per 64 pixels and rays shared
-def test_deflection_is_rounded_before_the_subtraction(tmp_path, monkeypatch, axis, n):
-    (tmp_path / "linear.cl").write_text(LENS)
+def test_deflection_is_rounded_before_the_subtraction(tmp_path, monkeypatch, axis, form, n):
+    (tmp_path / "linear.cl").write_text(LENS % form)
     (tmp_path / "position.cl").write_text(SOURCE % axis)
     monkeypatch.setenv("LENSED_OBJECTS_PATH", str(tmp_path))
     shape = (40, 56)
