@@ -95,10 +95,14 @@ std::string model_source(const std::vector<std::vector<ModelObject>>& models, st
           << "const float4* cc, float rho) { return cull_" << k << "(data, base, tab, cc, rho); }\n"
           << "template <> inline void cull_consts_model<" << k << ">(uint* data, float4* cc) "
           << "{ cull_consts_" << k << "(data, cc); }\n";
-    o << "constexpr bool model_holds(int k) { return false";
-    for (size_t k = 0; k < models.size(); ++k)
-        if (model_holds(models[k])) o << " || k == " << k;
-    o << "; }\n";
+    auto lists = [&](const char* name, bool (*which)(const std::vector<ModelObject>&)) {
+        o << "constexpr bool " << name << "(int k) { return false";
+        for (size_t k = 0; k < models.size(); ++k)
+            if (which(models[k])) o << " || k == " << k;
+        o << "; }\n";
+    };
+    lists("model_holds", model_holds);
+    lists("model_tabulates", model_tabulates);
     o << "}  // namespace lcl\n#ifdef LCL_GPU\n#pragma clang force_cuda_host_device end\n#endif\n";
     return o.str();
 }

@@ -400,6 +400,10 @@ bool model_adds_exps(const std::vector<ModelObject>& objs) {
     return n > 1;
 }
 
+bool model_tabulates(const std::vector<ModelObject>& objs) {
+    return std::any_of(objs.begin(), objs.end(), [](const ModelObject& ob) { return ob.table; });
+}
+
 bool model_holds(const std::vector<ModelObject>& objs) {
     // at most 64 words, so that the block and the ray's own values (about 50
     // registers with two sources) stay within the loop's 128 registers

@@ -70,6 +70,8 @@ bool model_culls(const std::vector<ModelObject>& objs);
 bool model_adds_exps(const std::vector<ModelObject>& objs);
 // whether the render holds the model's data block in vector registers
 bool model_holds(const std::vector<ModelObject>& objs);
+// whether a lens of the model has a table
+bool model_tabulates(const std::vector<ModelObject>& objs);
 std::string set_params_function(const std::vector<ModelObject>& objs, int k);
 
 // Total data words of a model.

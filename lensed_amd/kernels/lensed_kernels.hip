@@ -312,8 +312,10 @@ extern "C" __global__ __launch_bounds__(LENSED_RENDER_BS) __attribute__((amdgpu_
 // one after the other, so one candidate's image takes the latency of 49 rays
 // in a row on a few waves.  Here each ray's value goes to LDS and
 // the first wave adds them up in node order with the same operations as
-// lensed_render, so the bits are the same.
-template <int K, bool ERR>
+// lensed_render, so the bits are the same.  (One form for both uses: the error
+// plane's sum is not the rays' work, and a second form of them takes the
+// compiler as long as lensed_render does.)
+template <int K>
 __device__ inline void lensed_render_wide_item(const lensed_desc& d, int cand, int px, int py, bool on, bool restage,
                                                const u32* __restrict__ blocks, const float4* __restrict__ quad,
                                                const float4* __restrict__ tables, const float4* __restrict__ npre,
@@ -366,11 +368,11 @@ __device__ inline void lensed_render_wide_item(const lensed_desc& d, int cand, i
             const float4 node = q[n];
             const float v = rays[n * 64 + lane];
             f = __builtin_fmaf(node.z, v, f);
-            if (ERR) e = __builtin_fmaf(node.w, v, e);
+            e = __builtin_fmaf(node.w, v, e);
         }
         const long long o = d.model_off + (long long)cand * d.npix + py * d.width + px;
         model[o] = f;
-        if (ERR) errp[o] = e;
+        if (errp) errp[o] = e;
     }
     __syncthreads();  // the next unit writes the rays again
 }
@@ -412,12 +414,8 @@ extern "C" __global__ __launch_bounds__(LENSED_RENDER_BS) __attribute__((amdgpu_
         switch (d.model) {
 #define LENSED_WIDE_CASE(K)                                                                                     \
     case K:                                                                                                     \
-        if (errp)                                                                                               \
-            lensed_render_wide_item<K, true>(d, cand, px, py, on, restage, blocks, quad, tables, npre, tab_lds, \
-                                             rays, model, errp);                                                \
-        else                                                                                                    \
-            lensed_render_wide_item<K, false>(d, cand, px, py, on, restage, blocks, quad, tables, npre,         \
-                                              tab_lds, rays, model, errp);                                      \
+        lensed_render_wide_item<K>(d, cand, px, py, on, restage, blocks, quad, tables, npre, tab_lds, rays,     \
+                                   model, errp);                                                                \
         break;
             LENSED_FOR_MODELS(LENSED_WIDE_CASE)
 #undef LENSED_WIDE_CASE
@@ -744,8 +742,10 @@ __device__ __attribute__((always_inline)) inline void lensed_epl_tables_block(
         switch (d.model) {
 #define LENSED_PAIRS_CASE(K)                                                          \
     case K:                                                                           \
-        lcl::set_params_##K(blk, p);                                                  \
-        lensed_node_pairs<K>(d, blk, quad, npre, cand, i, LENSED_EPL_NT);             \
+        if constexpr (lcl::model_tabulates(K)) {                                      \
+            lcl::set_params_##K(blk, p);                                              \
+            lensed_node_pairs<K>(d, blk, quad, npre, cand, i, LENSED_EPL_NT);         \
+        }                                                                             \
         break;
             LENSED_FOR_MODELS(LENSED_PAIRS_CASE)
 #undef LENSED_PAIRS_CASE
