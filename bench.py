@@ -628,7 +628,7 @@ def main():
                           "path": "batched, per-ray tenth-order EPL series"},
         "accuracy_vs_exact": acc,
         "plain_gpu": {"value": round(plain_rate, 2), "unit": "logL evals/s",
-                      "path": "one candidate per loglike() call, 4 kernels + sync, parameters and logL through pinned memory",
+                      "path": "one candidate per loglike() call, 3 kernels + sync, parameters and logL through pinned memory",
                       "identical_logL_to_batched": same},
         "speedup_vs_plain": round(value / plain_rate, 3),
         "roofline": render_roofline(kt, tr, K),
