@@ -272,11 +272,41 @@ static std::string without_comments(const std::string& src) {
     return out;
 }
 
-// whether a plugin defines the functions named by the patterns
-static bool plugin_defines(const std::string& name, const std::vector<const char*>& patterns) {
+// where the code from `at` on names `word` and opens a parenthesis, or npos
+static size_t find_call(const std::string& src, const std::string& word, size_t at = 0) {
+    for (size_t i = src.find(word, at); i != std::string::npos; i = src.find(word, i + 1)) {
+        size_t j = i + word.size();
+        if (i > 0 && is_ident_char(src[i - 1])) continue;
+        while (j < src.size() && isspace((unsigned char)src[j])) ++j;
+        if (j < src.size() && src[j] == '(') return i;
+    }
+    return std::string::npos;
+}
+
+struct Function {
+    const char *type, *name;
+};
+
+// whether a plugin defines the functions, each as "static type name("
+static bool plugin_defines(const std::string& name, const std::vector<Function>& functions) {
     const std::string src = without_comments(plugin_text(name));
+    // the word that ends before i, white space between; i moves to its start
+    auto before = [&](size_t& i, const std::string& word) {
+        const size_t end = i;
+        while (i > 0 && isspace((unsigned char)src[i - 1])) --i;
+        if (i == end || i < word.size() || src.compare(i - word.size(), word.size(), word) != 0) return false;
+        i -= word.size();
+        return true;
+    };
     bool ok = !src.empty();
-    for (const char* re : patterns) ok = ok && std::regex_search(src, std::regex(re));
+    for (const Function& f : functions) {
+        bool found = false;
+        for (size_t at = find_call(src, f.name); !found && at != std::string::npos; at = find_call(src, f.name, at + 1)) {
+            size_t i = at;
+            found = before(i, f.type) && before(i, "static");
+        }
+        ok = ok && found;
+    }
     return ok;
 }
 
@@ -301,12 +331,11 @@ bool object_table_shear(const std::string& name) {
 }
 
 static bool source_has_frame(const std::string& name) {
-    return plugin_defines(name, {R"(static\s+float2\s+frame_centre\s*\()", R"(static\s+float2\s+frame_map\s*\()",
-                                 R"(static\s+float\s+frame_profile\s*\()"});
+    return plugin_defines(name, {{"float2", "frame_centre"}, {"float2", "frame_map"}, {"float", "frame_profile"}});
 }
 
 static bool source_has_cutoff(const std::string& name) {
-    return plugin_defines(name, {R"(static\s+float\s+frame_cutoff\s*\()"});
+    return plugin_defines(name, {{"float", "frame_cutoff"}});
 }
 
 // The lens-frame form of a tabulated EPL lens applies when that lens is the
@@ -332,9 +361,9 @@ static int frame_source(const std::vector<ModelObject>& objs) {
 // fuses with
 static bool ends_in_sum(const std::string& name) {
     const std::string src = without_comments(plugin_text(name));
-    std::smatch m;
-    if (!std::regex_search(src, m, std::regex(R"(static\s+float2\s+deflection\s*\()"))) return false;
-    const size_t b = m.position(0), e = src.find("\n}", b);
+    const size_t b = find_call(src, "deflection");
+    if (b == std::string::npos) return false;
+    const size_t e = src.find("\n}", b);
     const std::string body = src.substr(b, e == std::string::npos ? e : e - b);
     auto blank = [&](size_t& i) { while (i < body.size() && isspace((unsigned char)body[i])) ++i; };
     int n = 0;
@@ -385,9 +414,9 @@ static bool slope_culls(const std::vector<ModelObject>& objs) {
     for (size_t i = 0; i < objs.size(); ++i) {
         const std::string& name = objs[i].name;
         if (i < nlens) {
-            if (objs[i].table || !plugin_defines(name, {R"(static\s+float\s+deflection_slope\s*\()"})) return false;
+            if (objs[i].table || !plugin_defines(name, {{"float", "deflection_slope"}})) return false;
         } else if (objs[i].type != OBJ_SOURCE || !source_has_frame(name) || !source_has_cutoff(name) ||
-                   !plugin_defines(name, {R"(static\s+bool\s+frame_compact\s*\()"})) {
+                   !plugin_defines(name, {{"bool", "frame_compact"}})) {
             return false;
         }
     }
@@ -396,7 +425,8 @@ static bool slope_culls(const std::vector<ModelObject>& objs) {
 
 bool model_adds_exps(const std::vector<ModelObject>& objs) {
     int n = 0;
-    for (const auto& ob : objs) n += ob.type == OBJ_SOURCE && plugin_defines(ob.name, {R"(\bexp\s*\()"});
+    for (const auto& ob : objs)
+        n += ob.type == OBJ_SOURCE && find_call(without_comments(plugin_text(ob.name)), "exp") != std::string::npos;
     return n > 1;
 }
 
