@@ -50,7 +50,8 @@ def run(tmp_path_factory):
                            os.path.join(HERE, "hip_stub.cpp")])
 
     def call(code):
-        env = dict(os.environ, LD_PRELOAD=so, LENSED_CACHE_DIR=str(d))
+        preload = ":".join(p for p in (so, os.environ.get("LD_PRELOAD")) if p)
+        env = dict(os.environ, LD_PRELOAD=preload, LENSED_CACHE_DIR=str(d))
         r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(code)], env=env, capture_output=True,
                            text=True, timeout=300)
         assert r.returncode == 0, (r.returncode, r.stderr[-3000:])
