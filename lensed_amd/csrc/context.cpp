@@ -326,7 +326,7 @@ static int build_layout(::lensed* l, const std::vector<size_t>& ncand, Layout& L
     // 108, 60, 67.  Of 160, a fifth more, 8192: 966, 797, 686 and 144, 69, 68;
     // 13 x 13 taps 16384: 335, 144, 149.  Images of at most four rows don't
     // count, what they fill of a tile of either height is next to nothing:
-    // 600 of 1 x 70, 3 x 3 taps: 7.7, 9.5, 12.1)
+    // 1200 of 1 x 64, 3 x 3 taps: 7.7, 9.5, 12.1)
     long long n32 = 0, n64 = 0, r32 = 0, r64 = 0;
     long long per_cu = 2;  // tall tiles the launch has to have
     double grown = 1.4;    // rows in tall tiles to rows in 32-row ones, below this
@@ -1087,7 +1087,7 @@ lensed* lensed_create(const lensed_system* systems, size_t nsys, const lensed_op
         // an SIE's, its bound as much again) gains nothing there.  (us a call,
         // culled and not, without a table, sigma 1/8 of the Einstein radius:
         // EPL + shear 16 x 16 4375 candidates 273, 223; 24 x 24 1500: 170,
-        // 150; 32 x 32 262: 90, 74; 40 x 40 1333: 230, 288; SIE 16 x 16 4375:
+        // 150; 32 x 32 262: 90, 74; 48 x 48 1333: 286, 323; SIE 16 x 16 4375:
         // 345, 300; 24 x 24 262: 86, 98; 32 x 32 193: 94, 97; 3000: 569, 539)
         if (S.cull && !S.table) {
             for (const auto& ob : S.objs) S.series = S.series || (ob.type == OBJ_LENS && object_tabulates(ob.name));
